@@ -428,9 +428,9 @@ int pm_mg_resnorm(pm_mg* mg, void* phi, const void* rhs, double* out_host, pm_st
  * valid extents sizes[3b..3b+2] (box-local indices from 0) and `ghost` ghost
  * layers; ghosted storage holds the boxes one after another (x fastest over
  * [-ghost, n+ghost)), valid storage likewise over [0, n).  Each operator is
- * ONE persistent launch over all boxes (a work queue of tiles, largest first)
- * instead of Proto's launch per box (e.g. LevelMultigridSolverImplem.H:
- * 366-378); the queue resets itself, so the launch can be graph-captured. */
+ * ONE launch over all boxes (a table of tiles, or a work queue that resets
+ * itself) instead of Proto's launch per box (e.g. LevelMultigridSolverImplem.H:
+ * 366-378), so it can be graph-captured. */
 typedef struct pm_batch pm_batch;
 int pm_batch_create(pm_batch** out, int nboxes, const int* sizes_host, int ghost);
 int pm_batch_destroy(pm_batch* batch);
@@ -438,8 +438,9 @@ int pm_batch_elems(const pm_batch* batch, size_t* ghosted, size_t* valid);
 /* nboxes + 1 element offsets of every box in ghosted / valid storage. */
 int pm_batch_offsets(const pm_batch* batch, size_t* ghosted_off, size_t* valid_off);
 /* Tiling knobs of the batched operators (what pm_batch_autotune searches):
- * z planes per apply tile (0 = whole box), persistent workgroups per CU for
- * the apply, rows per GSRB tile (fewer when an FP64 tile as wide as the widest
+ * z planes per apply tile (0 = whole box; until pm_batch_configure sets it,
+ * chosen from the batch's size), workgroups per CU for the apply (accepted and
+ * kept, but without effect: the apply runs one workgroup per tile), rows per GSRB tile (fewer when an FP64 tile as wide as the widest
  * box would not fit the 64 KiB LDS of a workgroup), workgroups per CU for
  * the sweep. */
 typedef struct pm_batch_config {

@@ -1,12 +1,13 @@
-// Batches of independent patches of uneven size (AMR boxes): one persistent
-// launch per operator for the whole batch.
+// Batches of independent patches of uneven size (AMR boxes): one launch per
+// operator for the whole batch.
 //
 // Proto applies an operator to a set of boxes as one launch per box
 // (`for (auto iter : layout) ...`, e.g. Proto_LevelMultigridSolverImplem.H:
-// 366-378).  Here a fixed grid of workgroups pulls tiles of every box from an
-// atomic work queue (largest tiles first); the queue counters reset
-// themselves at the end of each launch, so the launch can be captured in a
-// hipGraph and replayed without a memset node.
+// 366-378).  The apply and the row sweeps launch one workgroup per tile, the
+// tile read from a table by blockIdx.x.  In the LDS-ring sweep a fixed grid of
+// workgroups pulls tiles of every box from an atomic work queue (largest tiles
+// first); the queue counters reset themselves at the end of each launch, so
+// the launch can be captured in a hipGraph and replayed without a memset node.
 //
 // Storage: box b (valid extents n = sizes[b], g ghost layers) at
 // ghosted_off[b] in the ghosted array (x fastest over [-g, n+g)) and at
@@ -38,11 +39,11 @@ struct pm_batch {
     std::vector<int> sizes;
     std::vector<size_t> goff, voff;  // nboxes + 1
     void* d_boxes = nullptr;         // BatchBox[nboxes]
-    void* d_items = nullptr;         // BatchItem[] (apply)
-    int nitems_apply = 0, apply_rows = 0, apply_tz = 0;
+    void* d_items = nullptr;         // BatchItem[] (apply), one workgroup each
+    int nitems_apply = 0, apply_tz = -1;  // apply_tz -1: the z chunk of apply_auto_zc
     void* d_gitems = nullptr;        // BatchItem[] (gsrb)
     int nitems_gsrb = 0, gsrb_rows = 0;
-    unsigned* d_counter = nullptr;   // 2 x (queue head, blocks done) per operator
+    unsigned* d_counter = nullptr;   // queue head, blocks done (LDS-ring sweep)
     pm_batch_config cfg{0, 4, 8, 4};
     // the row-register sweep: every box 2..64 cells wide (rows_ok), its items
     // built for rows_ry rows per sub-tile; sweep_form as pm_batch_sweep_form
@@ -112,114 +113,116 @@ __device__ inline void queue_done(unsigned* counter)
 // and a step's results are stored at the start of the next step, after its
 // loads: the only waits are at the LDS commits and cover operations a whole
 // step old.
+//
+// One workgroup per tile, its tile fixed by blockIdx.x: the dispatcher hands a
+// free slot the next workgroup, so no queue is needed.  What bounds it: small
+// batches, the z walk of a tile (about 0.5 us a plane), hence the short z
+// chunks of apply_auto_zc; large ones, issue (27 multiplies and adds a cell)
+// and HBM about equally.  27 points, FP64 / FP32, against the same tiles drawn
+// from an atomic queue by 4 workgroups a CU (whose counter alone took some
+// 30 us of a launch): 20 boxes 90 / 76 -> 10 / 7 us, 300 boxes 109 / 108 ->
+// 67 / 39, 2000 boxes (mean 54 000 cells) 500 / 272 -> 460 / 217.
 constexpr int BA_RY = 4, BA_NL = 5, BA_NP = 256 * BA_NL;
 
 template<typename T, int SHAPE, int NT>
 __global__ __launch_bounds__(256) void k_batch_apply(const BatchBox* __restrict__ boxes,
-                                                     const BatchItem* __restrict__ items, int nitems, int g,
-                                                     const T* __restrict__ src, T* __restrict__ dst, BCoefs<T> c,
-                                                     unsigned* counter)
+                                                     const BatchItem* __restrict__ items, int g,
+                                                     const T* __restrict__ src, T* __restrict__ dst, BCoefs<T> c)
 {
     constexpr int NC = SHAPE == 7 ? 7 : 27, RY = BA_RY, NL = BA_NL;
     __shared__ T sm[3][BA_NP];
-    __shared__ int s_item;
     const int tid = threadIdx.x;
-    for (;;) {
-        const int it = next_item(counter, &s_item);
-        if (it >= nitems) { break; }
-        const BatchItem wi = items[it];
-        const BatchBox bx = boxes[wi.box];
-        const int XW = wi.xw, TR = wi.rows, LX = XW + 2, NE = (TR * RY + 2) * LX;
-        const long Gx = bx.nx + 2 * g, Gxy = Gx * (bx.ny + 2 * g);
-        const T* s = src + bx.goff;
-        T* d = dst + bx.voff;
-        const int col = tid % XW, trow = tid / XW;
-        const bool tact = trow < TR;
-        const int x = wi.x0 + col, yb = wi.y0 + trow * RY;
-        int eoff[NL];
+    const BatchItem wi = items[blockIdx.x];
+    const BatchBox bx = boxes[wi.box];
+    const int XW = wi.xw, TR = wi.rows, LX = XW + 2, NE = (TR * RY + 2) * LX;
+    const long Gx = bx.nx + 2 * g, Gxy = Gx * (bx.ny + 2 * g);
+    const T* s = src + bx.goff;
+    T* d = dst + bx.voff;
+    const int col = tid % XW, trow = tid / XW;
+    const bool tact = trow < TR;
+    const int x = wi.x0 + col, yb = wi.y0 + trow * RY;
+    int eoff[NL];
 #pragma unroll
-        for (int k = 0; k < NL; k++) {
-            const int e = min(tid + 256 * k, NE - 1);
-            const int er = e / LX, ec = e - er * LX;
-            const int gx = wi.x0 - 1 + ec, gy = min(wi.y0 - 1 + er, bx.ny + g - 1);
-            eoff[k] = (gx + g) + (int)Gx * (gy + g);
-        }
-        T P[3][NL];
-        auto gload = [&](T (&p)[NL], int z) {
-            const T* base = s + Gxy * (long)(z + g);
-#pragma unroll
-            for (int k = 0; k < NL; k++) { p[k] = base[eoff[k]]; }
-        };
-        auto lstore = [&](const T (&p)[NL], T* pl) {
-#pragma unroll
-            for (int k = 0; k < NL; k++) { pl[tid + 256 * k] = p[k]; }
-        };
-        T q[3][RY + 2][3];
-        const int lr0 = tact ? trow * RY : 0;  // idle threads read row 0 (never stored)
-        auto lread = [&](T (&qq)[RY + 2][3], const T* pl) {
-#pragma unroll
-            for (int r = 0; r < RY + 2; r++)
-#pragma unroll
-                for (int cc = 0; cc < 3; cc++) { qq[r][cc] = pl[(lr0 + r) * LX + col + cc]; }
-        };
-        T res[RY];
-        int zres = -1;  // plane of the results held in res (-1: none)
-        auto put_res = [&]() {
-            if (zres < 0 || !tact) { return; }
-            T* o = d + x + (long)bx.nx * ((long)yb + (long)bx.ny * zres);
-#pragma unroll
-            for (int r = 0; r < RY; r++) {
-                if (yb + r < bx.ny) {
-                    if (NT) { __builtin_nontemporal_store(res[r], o + (long)r * bx.nx); } else { o[(long)r * bx.nx] = res[r]; }
-                }
-            }
-        };
-        // one z step: stage plane zz (slot S), store the previous step's
-        // results, emit plane zz - 1 from slots S+1 (zz-2), S+2 (zz-1), S (zz)
-        auto step = [&](auto sc, int zz) {
-            constexpr int S = decltype(sc)::value, SB = (S + 1) % 3, SC = (S + 2) % 3;
-            lstore(P[S], sm[S]);
-            gload(P[(S + 1) % 3], min(zz + 1, wi.z1));
-            put_res();
-            __syncthreads();
-            lread(q[S], sm[S]);
-#pragma unroll
-            for (int r = 0; r < RY; r++) {
-                auto tap = [&](int dx, int dy, int dz) -> T {
-                    return dz < 0 ? q[SB][r + 1 + dy][1 + dx]
-                                  : (dz == 0 ? q[SC][r + 1 + dy][1 + dx] : q[S][r + 1 + dy][1 + dx]);
-                };
-                T acc = 0;
-#pragma unroll
-                for (int j = 0; j < NC; j++) {
-                    acc = acc + c.c[j] * tap(shape_off<SHAPE>(j, 0), shape_off<SHAPE>(j, 1), shape_off<SHAPE>(j, 2));
-                }
-                res[r] = acc;
-            }
-            zres = zz - 1;
-        };
-        // planes z0 - 1 and z0: staged, nothing to emit yet
-        gload(P[0], wi.z0 - 1);
-        lstore(P[0], sm[0]);
-        gload(P[1], wi.z0);
-        __syncthreads();
-        lread(q[0], sm[0]);
-        lstore(P[1], sm[1]);
-        gload(P[2], min(wi.z0 + 1, wi.z1));
-        __syncthreads();
-        lread(q[1], sm[1]);
-        int zz = wi.z0 + 1;
-        for (;;) {
-            step(std::integral_constant<int, 2>{}, zz);
-            if (++zz > wi.z1) { break; }
-            step(std::integral_constant<int, 0>{}, zz);
-            if (++zz > wi.z1) { break; }
-            step(std::integral_constant<int, 1>{}, zz);
-            if (++zz > wi.z1) { break; }
-        }
-        put_res();
+    for (int k = 0; k < NL; k++) {
+        const int e = min(tid + 256 * k, NE - 1);
+        const int er = e / LX, ec = e - er * LX;
+        const int gx = wi.x0 - 1 + ec, gy = min(wi.y0 - 1 + er, bx.ny + g - 1);
+        eoff[k] = (gx + g) + (int)Gx * (gy + g);
     }
-    queue_done(counter);
+    T P[3][NL];
+    auto gload = [&](T (&p)[NL], int z) {
+        const T* base = s + Gxy * (long)(z + g);
+#pragma unroll
+        for (int k = 0; k < NL; k++) { p[k] = base[eoff[k]]; }
+    };
+    auto lstore = [&](const T (&p)[NL], T* pl) {
+#pragma unroll
+        for (int k = 0; k < NL; k++) { pl[tid + 256 * k] = p[k]; }
+    };
+    T q[3][RY + 2][3];
+    const int lr0 = tact ? trow * RY : 0;  // idle threads read row 0 (never stored)
+    auto lread = [&](T (&qq)[RY + 2][3], const T* pl) {
+#pragma unroll
+        for (int r = 0; r < RY + 2; r++)
+#pragma unroll
+            for (int cc = 0; cc < 3; cc++) { qq[r][cc] = pl[(lr0 + r) * LX + col + cc]; }
+    };
+    T res[RY];
+    int zres = -1;  // plane of the results held in res (-1: none)
+    auto put_res = [&]() {
+        if (zres < 0 || !tact) { return; }
+        T* o = d + x + (long)bx.nx * ((long)yb + (long)bx.ny * zres);
+#pragma unroll
+        for (int r = 0; r < RY; r++) {
+            if (yb + r < bx.ny) {
+                if (NT) { __builtin_nontemporal_store(res[r], o + (long)r * bx.nx); } else { o[(long)r * bx.nx] = res[r]; }
+            }
+        }
+    };
+    // one z step: stage plane zz (slot S), store the previous step's
+    // results, emit plane zz - 1 from slots S+1 (zz-2), S+2 (zz-1), S (zz)
+    auto step = [&](auto sc, int zz) {
+        constexpr int S = decltype(sc)::value, SB = (S + 1) % 3, SC = (S + 2) % 3;
+        lstore(P[S], sm[S]);
+        gload(P[(S + 1) % 3], min(zz + 1, wi.z1));
+        put_res();
+        __syncthreads();
+        lread(q[S], sm[S]);
+#pragma unroll
+        for (int r = 0; r < RY; r++) {
+            auto tap = [&](int dx, int dy, int dz) -> T {
+                return dz < 0 ? q[SB][r + 1 + dy][1 + dx]
+                              : (dz == 0 ? q[SC][r + 1 + dy][1 + dx] : q[S][r + 1 + dy][1 + dx]);
+            };
+            T acc = 0;
+#pragma unroll
+            for (int j = 0; j < NC; j++) {
+                acc = acc + c.c[j] * tap(shape_off<SHAPE>(j, 0), shape_off<SHAPE>(j, 1), shape_off<SHAPE>(j, 2));
+            }
+            res[r] = acc;
+        }
+        zres = zz - 1;
+    };
+    // planes z0 - 1 and z0: staged, nothing to emit yet
+    gload(P[0], wi.z0 - 1);
+    lstore(P[0], sm[0]);
+    gload(P[1], wi.z0);
+    __syncthreads();
+    lread(q[0], sm[0]);
+    lstore(P[1], sm[1]);
+    gload(P[2], min(wi.z0 + 1, wi.z1));
+    __syncthreads();
+    lread(q[1], sm[1]);
+    int zz = wi.z0 + 1;
+    for (;;) {
+        step(std::integral_constant<int, 2>{}, zz);
+        if (++zz > wi.z1) { break; }
+        step(std::integral_constant<int, 0>{}, zz);
+        if (++zz > wi.z1) { break; }
+        step(std::integral_constant<int, 1>{}, zz);
+        if (++zz > wi.z1) { break; }
+    }
+    put_res();
 }
 
 // ------------------------------------------------------------ batched GSRB
@@ -400,9 +403,14 @@ __global__ __launch_bounds__(256) void k_batch_gsrb(const BatchBox* __restrict__
 // (each lane also loads its own edge neighbour, or itself, per row).  Ghost
 // rows and planes are loaded (clamped into the ghosted box) but never updated
 // or written.  Lanes past the last sub-tile shadow lane 0 and store nothing.
+// An item sweeps planes [z0, z1): it starts two planes below z0 (the red cells
+// of plane z0 - 1, recomputed, are the black cells' neighbours) and writes from
+// z0 on.
 struct RowItem {
-    int box, y0, nsub, pad;
+    int box, y0, nsub, z0, z1;
 };
+// The first step of an item: plane -1 at the bottom of a box, else z0 - 2.
+__device__ inline int first_step(const RowItem& wi) { return wi.z0 == 0 ? -1 : wi.z0 - 2; }
 
 // waves per workgroup of the row and pair sweeps unless set otherwise (config
 // 4, 2000 boxes: FP32 row sweep 0.397 ms with 4 waves, 0.416 with 1, 0.513
@@ -418,7 +426,6 @@ __global__ __launch_bounds__(64 * WPB) void k_batch_rows(const BatchBox* __restr
     constexpr int NR = RY + 4;  // phi rows held: Y0 - 2 .. Y0 + RY + 1
     constexpr int NQ = RY + 2;  // rhs and edge rows: Y0 - 1 .. Y0 + RY
     const RowItem wi = items[blockIdx.x];
-    if (wi.box < 0) { return; }  // padding of a shorter XCD list
     const BatchBox bx = boxes[wi.box];
     const int nx = bx.nx, ny = bx.ny, nz = bx.nz;
     // wave w of the workgroup holds sub-tiles w P .. w P + P - 1 of the item
@@ -531,7 +538,7 @@ __global__ __launch_bounds__(64 * WPB) void k_batch_rows(const BatchBox* __restr
                 P[S1][i] = (((upd >> i) & 1u) && is_red(i, k + 1)) ? nv : cur;
             }
         }
-        if (k >= 0) {  // black cells of plane k, rows Y0 .. Y0 + RY - 1, then plane k out
+        if (k >= wi.z0) {  // black cells of plane k, rows Y0 .. Y0 + RY - 1, then plane k out
 #pragma unroll
             for (int r = 0; r < RY; r++) {
                 const int i = r + 2;
@@ -557,21 +564,21 @@ __global__ __launch_bounds__(64 * WPB) void k_batch_rows(const BatchBox* __restr
             }
         }
     };
-    // planes -1 .. PF (slots 0 .. PF + 1), rhs and edges of planes 0 .. PF - 1 (slots 1 .. PF)
-    static_for<0, PF + 2>([&](auto zc) { loadP(P[decltype(zc)::value], decltype(zc)::value - 1); });
+    // planes k .. k + 1 + PF (slots 0 .. PF + 1), rhs and edges of planes k + 1 .. k + PF (slots 1 .. PF)
+    int k = first_step(wi);
+    static_for<0, PF + 2>([&](auto zc) { loadP(P[decltype(zc)::value], k + decltype(zc)::value); });
     static_for<0, PF>([&](auto zc) {
-        constexpr int z = decltype(zc)::value;
-        loadQ(Q[z + 1], z);
-        loadE(E[z + 1], z);
-        loadG(G[z + 1], z);
+        constexpr int z = decltype(zc)::value + 1;
+        loadQ(Q[z], k + z);
+        loadE(E[z], k + z);
+        loadG(G[z], k + z);
     });
-    int k = -1;
     bool done = false;
     for (;;) {
         static_for<0, R>([&](auto sc) {
             if (!done) {
                 step(sc, k);
-                done = ++k >= nz;
+                done = ++k >= wi.z1;
             }
         });
         if (done) { break; }
@@ -610,7 +617,6 @@ __global__ __launch_bounds__(64 * WPB) void k_batch_rows2(const BatchBox* __rest
     constexpr int NQ = RY + 2;  // rhs and edge rows: Y0 - 1 .. Y0 + RY
     static_assert(RY % 2 == 0, "sub-tiles start on even rows");
     const RowItem wi = items[blockIdx.x];
-    if (wi.box < 0) { return; }  // padding of a shorter XCD list
     const BatchBox bx = boxes[wi.box];
     const int nx = bx.nx, ny = bx.ny, nz = bx.nz, h = nx >> 1;
     // wave w of the workgroup holds sub-tiles w npw .. w npw + npw - 1 of the item
@@ -744,7 +750,7 @@ __global__ __launch_bounds__(64 * WPB) void k_batch_rows2(const BatchBox* __rest
                 }
             }
         }
-        if (k >= 0) {
+        if (k >= wi.z0) {
 #pragma unroll
             for (int r = 0; r < RY; r++) {
                 const int i = r + 2;
@@ -782,34 +788,34 @@ __global__ __launch_bounds__(64 * WPB) void k_batch_rows2(const BatchBox* __rest
         }
     };
     using std::integral_constant;
-    loadP(A[0], B[0], -1);
-    loadP(A[1], B[1], 0);
-    loadP(A[2], B[2], 1);
-    loadQ(QA[1], QB[1], 0);
-    loadE(E[1], 0);
-    loadG(G[1], 0);
-    int k = -1;
+    int k = first_step(wi);  // odd: plane k + 1 has parity 0
+    loadP(A[0], B[0], k);
+    loadP(A[1], B[1], k + 1);
+    loadP(A[2], B[2], k + 2);
+    loadQ(QA[1], QB[1], k + 1);
+    loadE(E[1], k + 1);
+    loadG(G[1], k + 1);
     for (;;) {
         step(integral_constant<int, 0>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 1>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 2>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 3>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 4>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 0>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 1>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 2>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 3>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 4>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
     }
 }
 
@@ -840,7 +846,6 @@ __global__ __launch_bounds__(64) void k_batch_rows4(const BatchBox* __restrict__
     constexpr int NQ = RY + 2;  // rhs rows: Y0 - 1 .. Y0 + RY
     static_assert(RY % 2 == 0, "sub-tiles start on even rows");
     const RowItem wi = items[blockIdx.x];
-    if (wi.box < 0) { return; }  // padding of a shorter XCD list
     const BatchBox bx = boxes[wi.box];
     const int nx = bx.nx, ny = bx.ny, nz = bx.nz, h = (nx >> 2) + 1;
     const int lane = threadIdx.x & 63, npw = 64 / h;
@@ -951,7 +956,7 @@ __global__ __launch_bounds__(64) void k_batch_rows4(const BatchBox* __restrict__
                 }
             }
         }
-        if (k >= 0) {
+        if (k >= wi.z0) {
 #pragma unroll
             for (int r = 0; r < RY; r++) {
                 const int i = r + 2;
@@ -977,32 +982,32 @@ __global__ __launch_bounds__(64) void k_batch_rows4(const BatchBox* __restrict__
         }
     };
     using std::integral_constant;
-    loadP(P[0], -1);
-    loadP(P[1], 0);
-    loadP(P[2], 1);
-    loadQ(Q[1], 0);
-    int k = -1;
+    int k = first_step(wi);  // odd: plane k + 1 has parity 0
+    loadP(P[0], k);
+    loadP(P[1], k + 1);
+    loadP(P[2], k + 2);
+    loadQ(Q[1], k + 1);
     for (;;) {
         step(integral_constant<int, 0>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 1>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 2>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 3>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 4>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 0>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 1>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 2>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 3>{}, integral_constant<int, 0>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
         step(integral_constant<int, 4>{}, integral_constant<int, 1>{}, k);
-        if (++k >= nz) { break; }
+        if (++k >= wi.z1) { break; }
     }
 }
 
@@ -1027,30 +1032,90 @@ int upload(void** dptr, const void* host, size_t bytes)
     return PM_OK;
 }
 
-// Apply tiles: x in steps of 64; TR thread-rows of BA_RY rows each, TR the
-// largest with TR * XW <= 256 threads, TR * BA_RY no more than the rows left
-// (rounded up) and the staged plane (TR BA_RY + 2) (XW + 2) <= BA_NP; z chunks
-// of tz (0 = whole box); largest first.
+// Boxes spread over the 8 XCDs (workgroup w runs on XCD w mod 8) by cell count,
+// largest first, each to the least loaded, so that the tiles of a box share an
+// L2 that serves the halo rows they re-read.
+constexpr int kXcd = 8;
+std::vector<std::vector<int>> boxes_by_xcd(const pm_batch* B)
+{
+    std::vector<int> order(B->nboxes);
+    for (int b = 0; b < B->nboxes; b++) { order[b] = b; }
+    auto cells = [&](int b) { return (long)B->sizes[3 * b] * B->sizes[3 * b + 1] * B->sizes[3 * b + 2]; };
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cells(a) > cells(b); });
+    std::vector<std::vector<int>> xb(kXcd);
+    std::vector<long> load(kXcd, 0);
+    for (int b : order) {
+        const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+        xb[x].push_back(b);
+        load[x] += cells(b);
+    }
+    return xb;
+}
+
+// The launch order of per-XCD item lists: one item of each list in turn, so
+// that item m of list x lands on XCD x; where a list has ended the others
+// take its turns (a batch of few boxes then still reaches every XCD).
+template<typename Item>
+std::vector<Item> interleave(const std::vector<std::vector<Item>>& lists)
+{
+    std::vector<Item> items;
+    size_t nmax = 0;
+    for (const auto& l : lists) { nmax = std::max(nmax, l.size()); }
+    for (size_t m = 0; m < nmax; m++)
+        for (const auto& l : lists) {
+            if (m < l.size()) { items.push_back(l[m]); }
+        }
+    return items;
+}
+
+// The x-y tiles of box b of the apply, f(x0, xw, y0, tr): x in steps of 64; TR
+// thread-rows of BA_RY rows each, TR the largest with TR * XW <= 256 threads,
+// TR * BA_RY no more than the rows left (rounded up) and the staged plane
+// (TR BA_RY + 2) (XW + 2) <= BA_NP.
+template<typename F>
+void apply_tiles(const pm_batch* B, int b, F&& f)
+{
+    const int nx = B->sizes[3 * b], ny = B->sizes[3 * b + 1];
+    for (int x0 = 0; x0 < nx; x0 += 64) {
+        const int xw = std::min(64, nx - x0);
+        const int trmax = std::max(1, std::min(256 / xw, (BA_NP / (xw + 2) - 2) / BA_RY));
+        for (int y0 = 0; y0 < ny; y0 += trmax * BA_RY) {
+            f(x0, xw, y0, std::min(trmax, (ny - y0 + BA_RY - 1) / BA_RY));
+        }
+    }
+}
+
+// Automatic z chunk of the apply: about four workgroups per CU over the batch,
+// at least 4 planes (a chunk stages two more than it writes) and at most 24.
+// 27 points, FP32: 20 boxes 7 us with 4 planes, 51 with whole boxes; 300 boxes
+// 35 with 8, 57 whole; 2000 boxes 224 with 24, 243 whole, 274 with 4.
+int apply_auto_zc(const pm_batch* B)
+{
+    long planes = 0;  // tile planes of the whole batch
+    for (int b = 0; b < B->nboxes; b++) {
+        apply_tiles(B, b, [&](int, int, int, int) { planes += B->sizes[3 * b + 2]; });
+    }
+    return (int)std::min(24L, std::max(4L, planes / 1024));
+}
+
+// Apply items: the tiles of every box in z chunks of tz (0 = whole box, -1 =
+// apply_auto_zc).  Each XCD's list takes its boxes largest first.
 int build_apply_items(pm_batch* B, int tz)
 {
-    std::vector<BatchItem> items;
-    for (int b = 0; b < B->nboxes; b++) {
-        const int nx = B->sizes[3 * b], ny = B->sizes[3 * b + 1], nz = B->sizes[3 * b + 2];
-        for (int x0 = 0; x0 < nx; x0 += 64) {
-            const int xw = std::min(64, nx - x0);
-            const int trmax = std::max(1, std::min(256 / xw, (BA_NP / (xw + 2) - 2) / BA_RY));
-            for (int y0 = 0; y0 < ny; y0 += trmax * BA_RY) {
-                const int tr = std::min(trmax, (ny - y0 + BA_RY - 1) / BA_RY);
-                const int zc = tz > 0 ? tz : nz;
-                for (int z0 = 0; z0 < nz; z0 += zc) {
-                    items.push_back(BatchItem{b, x0, y0, z0, std::min(nz, z0 + zc), tr, xw, 0});
-                }
+    const int zauto = tz < 0 ? apply_auto_zc(B) : tz;
+    const auto xb = boxes_by_xcd(B);
+    std::vector<std::vector<BatchItem>> lists(kXcd);
+    for (int x = 0; x < kXcd; x++) {
+        for (int b : xb[x]) {
+            const int nz = B->sizes[3 * b + 2], zc = zauto > 0 ? zauto : nz;
+            for (int z0 = 0; z0 < nz; z0 += zc) {
+                apply_tiles(B, b, [&](int x0, int xw, int y0, int tr) {
+                    lists[x].push_back(BatchItem{b, x0, y0, z0, std::min(nz, z0 + zc), tr, xw, 0});
+                });
             }
         }
     }
-    std::stable_sort(items.begin(), items.end(), [](const BatchItem& a, const BatchItem& b) {
-        return (long)a.xw * a.rows * (a.z1 - a.z0) > (long)b.xw * b.rows * (b.z1 - b.z0);
-    });  // rows = thread-rows: proportional to the tile's cells
+    const std::vector<BatchItem> items = interleave(lists);
     B->nitems_apply = (int)items.size();
     B->apply_tz = tz;
     return upload(&B->d_items, items.data(), sizeof(BatchItem) * items.size());
@@ -1095,42 +1160,44 @@ int build_gsrb_items(pm_batch* B, int rows)
 // wave (nx, nx / 2 lanes with one or two cells per lane; nx / 4 + 1 with four,
 // whose rows include the two ghost columns on each side), wpb waves per workgroup (one item each; the waves of an item
 // walk z together, so the halo rows they share are re-read while still
-// cached).  Workgroup w runs on XCD w mod 8, and
-// the strips of a box share halo rows, so every box goes whole to one XCD
-// (whose L2 then serves the re-read rows): boxes are spread over the 8 XCDs
-// by cell count (largest first, to the least loaded), each XCD's list takes
-// its boxes longest z extent first, and the lists are interleaved into the
-// launch order, shorter ones padded with empty items (box -1).
+// cached).  The strips of a box share halo rows, so every box goes whole to
+// one XCD (boxes_by_xcd), whose list takes its boxes longest z extent first.
 int build_row_items(pm_batch* B, int ry, int cpl, int wpb)
 {
-    constexpr int kXcd = 8;
-    std::vector<int> order(B->nboxes);
-    for (int b = 0; b < B->nboxes; b++) { order[b] = b; }
-    auto cells = [&](int b) { return (long)B->sizes[3 * b] * B->sizes[3 * b + 1] * B->sizes[3 * b + 2]; };
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cells(a) > cells(b); });
-    std::vector<std::vector<int>> xb(kXcd);
-    std::vector<long> load(kXcd, 0);
-    for (int b : order) {
-        const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        xb[x].push_back(b);
-        load[x] += cells(b);
+    auto xb = boxes_by_xcd(B);
+    auto per_item = [&](int b) {
+        const int nx = B->sizes[3 * b], lanes = cpl == 4 ? nx / 4 + 1 : nx / cpl;
+        return wpb * (64 / lanes);
+    };
+    // Planes per item: the whole box where that already gives about 1536 waves
+    // (six a CU; 3072 with one cell per lane, whose waves are shorter), else
+    // shorter chunks, which sweep three planes more than they write.  FP64 pairs
+    // (us, whole boxes -> chunks): 20 boxes 72 -> 10, 100 81 -> 31, 300 130 -> 116,
+    // from 600 boxes on whole; FP32 quads 42 -> 8, 43 -> 16, 47 -> 41.
+    long planes = 0;
+    for (int b = 0; b < B->nboxes; b++) {
+        const long nstrips = (B->sizes[3 * b + 1] + ry - 1) / ry, P = per_item(b);
+        planes += wpb * ((nstrips + P - 1) / P) * B->sizes[3 * b + 2];
     }
+    const int zc = (int)std::min(4096L, std::max(4L, planes / (cpl == 1 ? 3072 : 1536))) & ~1;
     std::vector<std::vector<RowItem>> lists(kXcd);
-    size_t nmax = 0;
     for (int x = 0; x < kXcd; x++) {
         std::stable_sort(xb[x].begin(), xb[x].end(),
                          [&](int a, int b) { return B->sizes[3 * a + 2] > B->sizes[3 * b + 2]; });
         for (int b : xb[x]) {
-            const int nx = B->sizes[3 * b], ny = B->sizes[3 * b + 1];
-            const int lanes = cpl == 4 ? nx / 4 + 1 : nx / cpl;
-            const int P = wpb * (64 / lanes), nstrips = (ny + ry - 1) / ry;
-            for (int s = 0; s < nstrips; s += P) { lists[x].push_back(RowItem{b, s * ry, std::min(P, nstrips - s), 0}); }
+            const int ny = B->sizes[3 * b + 1], nz = B->sizes[3 * b + 2];
+            const int P = per_item(b), nstrips = (ny + ry - 1) / ry;
+            // chunks start on plane 0 or an odd plane: the parity-unrolled walks begin two below
+            for (int z0 = 0; z0 < nz;) {
+                const int z1 = nz - z0 <= zc + 2 ? nz : (z0 == 0 ? zc + 1 : z0 + zc);
+                for (int s = 0; s < nstrips; s += P) {
+                    lists[x].push_back(RowItem{b, s * ry, std::min(P, nstrips - s), z0, z1});
+                }
+                z0 = z1;
+            }
         }
-        nmax = std::max(nmax, lists[x].size());
     }
-    std::vector<RowItem> items(nmax * kXcd, RowItem{-1, 0, 0, 0});
-    for (int x = 0; x < kXcd; x++)
-        for (size_t m = 0; m < lists[x].size(); m++) { items[m * kXcd + x] = lists[x][m]; }
+    const std::vector<RowItem> items = interleave(lists);
     if (cpl == 4) {
         B->nitems_quads = (int)items.size();
         return upload(&B->d_qitems, items.data(), sizeof(RowItem) * items.size());
@@ -1198,9 +1265,9 @@ int pm_batch_create(pm_batch** out, int nboxes, const int* sizes_host, int ghost
         B->voff[b + 1] = B->voff[b] + (size_t)nx * ny * nz;
     }
     int rc = upload(&B->d_boxes, boxes.data(), sizeof(BatchBox) * nboxes);
-    if (rc == PM_OK && hipMalloc((void**)&B->d_counter, 4 * sizeof(unsigned)) != hipSuccess) { rc = PM_ERR_NOMEM; }
-    if (rc == PM_OK && hipMemset(B->d_counter, 0, 4 * sizeof(unsigned)) != hipSuccess) { rc = PM_ERR_HIP; }
-    if (rc == PM_OK) { rc = build_apply_items(B, 0); }
+    if (rc == PM_OK && hipMalloc((void**)&B->d_counter, 2 * sizeof(unsigned)) != hipSuccess) { rc = PM_ERR_NOMEM; }
+    if (rc == PM_OK && hipMemset(B->d_counter, 0, 2 * sizeof(unsigned)) != hipSuccess) { rc = PM_ERR_HIP; }
+    if (rc == PM_OK) { rc = build_apply_items(B, -1); }
     if (rc == PM_OK) { rc = build_gsrb_items(B, B->cfg.gsrb_rows); }
     B->rows_ok = true;
     B->pairs_ok = ghost % 2 == 0;
@@ -1282,30 +1349,30 @@ int pm_batch_apply(pm_batch* B, const pm_stencil* st, const void* src, void* dst
     int rc = stencil_info(st, &kind, &dtype, &cv);
     if (rc) { return rc; }
     PM_REQUIRE(kind == 7 || kind == 27, "pm_batch_apply: needs the 7-point or 27-point Laplacian shape");
-    const unsigned nb = persistent_blocks(B->cfg.apply_blocks_per_cu);
+    const unsigned nb = (unsigned)B->nitems_apply;
     if (dtype == PM_F64) {
         BCoefs<double> cc;
         coefs_of<double>(cv, scale, cc);
         if (kind == 7) {
             hipLaunchKernelGGL((k_batch_apply<double, 7, 1>), dim3(nb), dim3(256), 0, S(stream),
-                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->nitems_apply, B->ghost,
-                               (const double*)src, (double*)dst, cc, B->d_counter);
+                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->ghost, (const double*)src,
+                               (double*)dst, cc);
         } else {
             hipLaunchKernelGGL((k_batch_apply<double, 27, 1>), dim3(nb), dim3(256), 0, S(stream),
-                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->nitems_apply, B->ghost,
-                               (const double*)src, (double*)dst, cc, B->d_counter);
+                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->ghost, (const double*)src,
+                               (double*)dst, cc);
         }
     } else {
         BCoefs<float> cc;
         coefs_of<float>(cv, scale, cc);
         if (kind == 7) {
             hipLaunchKernelGGL((k_batch_apply<float, 7, 1>), dim3(nb), dim3(256), 0, S(stream),
-                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->nitems_apply, B->ghost,
-                               (const float*)src, (float*)dst, cc, B->d_counter);
+                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->ghost, (const float*)src,
+                               (float*)dst, cc);
         } else {
             hipLaunchKernelGGL((k_batch_apply<float, 27, 1>), dim3(nb), dim3(256), 0, S(stream),
-                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->nitems_apply, B->ghost,
-                               (const float*)src, (float*)dst, cc, B->d_counter);
+                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->ghost, (const float*)src,
+                               (float*)dst, cc);
         }
     }
     PM_CHECK_LAUNCH();
@@ -1485,7 +1552,7 @@ int pm_batch_gsrb(pm_batch* B, int dtype, const void* phi_in, void* phi_out, con
         auto go = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(nb), dim3(256), lds, S(stream), (const BatchBox*)B->d_boxes,
                                (const BatchItem*)B->d_gitems, B->nitems_gsrb, B->ghost, (const T*)phi_in,
-                               (T*)phi_out, (const T*)rhs, coef, lamT, B->d_counter + 2, phi_elems);
+                               (T*)phi_out, (const T*)rhs, coef, lamT, B->d_counter, phi_elems);
         };
         if (np <= 1024) { go(k_batch_gsrb<T, 4>); }
         else if (np <= 2048) { go(k_batch_gsrb<T, 8>); }
@@ -1534,23 +1601,19 @@ int pm_batch_autotune(pm_batch* B, const pm_stencil* st, const void* src, void* 
         *ms /= (float)reps;
         return PM_OK;
     };
-    const int zs[] = {0, 8, 16, 32};
+    const int zs[] = {0, 8, 16, 32, apply_auto_zc(B)};
     const int bpcs[] = {1, 2, 4, 8};
     const int rows[] = {2, 4, 8, 16};
     pm_batch_config win = keep;
     float best_a = 1e30f, best_g = 1e30f;
     for (int z : zs) {
-        for (int bpc : bpcs) {
-            pm_batch_config c = keep;
-            c.apply_zplanes = z;
-            c.apply_blocks_per_cu = bpc;
-            rc = pm_batch_configure(B, &c);
-            float ms = 0;
-            if (rc == PM_OK) { rc = time([&]() { return pm_batch_apply(B, st, src, dst, 1.0, stream); }, &ms); }
-            if (rc) { break; }
-            if (ms < best_a) { best_a = ms; win.apply_zplanes = z; win.apply_blocks_per_cu = bpc; }
-        }
+        pm_batch_config c = keep;
+        c.apply_zplanes = z;
+        rc = pm_batch_configure(B, &c);
+        float ms = 0;
+        if (rc == PM_OK) { rc = time([&]() { return pm_batch_apply(B, st, src, dst, 1.0, stream); }, &ms); }
         if (rc) { break; }
+        if (ms < best_a) { best_a = ms; win.apply_zplanes = z; }
     }
     const size_t esz = dtype == PM_F64 ? 8 : 4;
     for (int r : rows) {

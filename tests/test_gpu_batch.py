@@ -333,3 +333,24 @@ def test_batch_gsrb_even_widths_vs_oracle(dt, ghost):
         p_out = dev(phi)
         B.gsrb(dt, vp(p_in), vp(p_out), vp(r_d), dx)
         assert first_diff(B, host(p_out), want, False) is None, (rows, first_diff(B, host(p_out), want, False))
+
+
+@pytest.mark.parametrize("dt", [pa.PM_F64, pa.PM_F32])
+@pytest.mark.parametrize("widths", [(16, 24), (14, 30), (15, 33)], ids=["quads", "pairs", "rows"])
+def test_batch_short_z_chunks_vs_oracle(dt, widths):
+    """A batch of a few boxes is cut into chunks of 4 planes (5 at the bottom of
+    a box, 4 to 6 at its top): every depth around the chunk edges, untuned, the
+    27-point apply and each row sweep's kernel."""
+    B = make_batch([(widths[i % 2], 9 + i % 4, nz) for i, nz in enumerate((1, 2, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 23))])
+    t = NPDT[dt]
+    coefs, offs, *_ = util.lib_stencil("Laplacian_27", 0, 3, t)
+    st = pa.Stencil(coefs, offs, dt)
+    src, rhs = inputs(B, dt, 31)
+    s_d, r_d, d_d, p_d = dev(src), dev(rhs), zeros(B.valid_elems, t), dev(src)
+    say("short z chunks", widths, dt)
+    B.apply(st, vp(s_d), vp(d_d), 0.37)
+    got, want = host(d_d), oracle_apply_batch(B, coefs, offs, src, 0.37)
+    assert first_diff(B, got, want, True) is None, first_diff(B, got, want, True)
+    B.gsrb(dt, vp(s_d), vp(p_d), vp(r_d), 1.0 / 32)
+    got, want = host(p_d), oracle_gsrb_batch(B, src, rhs, 1.0 / 32)
+    assert first_diff(B, got, want, False) is None, first_diff(B, got, want, False)
