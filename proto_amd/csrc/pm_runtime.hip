@@ -70,7 +70,9 @@ int workspace(hipStream_t stream, size_t bytes, void** out)
             w.bytes = 0;
             w.captured = false;
         }
-        size_t nb = bytes < ((size_t)1 << 16) ? ((size_t)1 << 16) : bytes;
+        // at least 96 KiB: the partials of a fused residual of up to about 200^3
+        // cells (3072 workgroups), so that a stream warmed by any call captures it
+        size_t nb = bytes < ((size_t)96 << 10) ? ((size_t)96 << 10) : bytes;
         hipError_t e = hipMalloc(&w.ptr, nb);
         if (e != hipSuccess) {
             set_error("workspace hipMalloc(%zu): %s", nb, hipGetErrorString(e));

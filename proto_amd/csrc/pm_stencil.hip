@@ -657,7 +657,49 @@ struct ZCfg {
     int ry, pf, nt, tz;  // rows per thread, planes prefetched, NT stores, planes per block (0: auto)
 };
 
-static ZCfg default_cfg(int dtype) { return ZCfg{dtype == PM_F64 ? 2 : 4, 1, 0, 0}; }
+// Workgroups of 64 x 4 ry x tz tiles over ibox.
+static long zblocks(const Box3& ibox, int ry, int tz)
+{
+    return ((box_nx(ibox) + 63) / 64) * ((box_ny(ibox) + 4 * ry - 1) / (4 * ry)) * ((box_nz(ibox) + tz - 1) / tz);
+}
+
+// Planes per workgroup where the configuration leaves them open: long runs
+// stage less halo (a run of tz stages tz + 2 planes), short ones reach all 256
+// CUs and end sooner (a plane takes a few hundred ns of load latency and
+// barriers).  16 where that still gives three workgroups a CU, then 8, then 4;
+// more than 16 only to keep the count of workgroups (and their partials)
+// bounded.
+static int auto_tz(const Box3& ibox, int ry)
+{
+    if (zblocks(ibox, ry, 16) >= 768) {
+        int tz = 16;
+        while (zblocks(ibox, ry, tz) > 16384 && tz < box_nz(ibox)) { tz *= 2; }
+        return tz;
+    }
+    return zblocks(ibox, ry, 8) >= 768 ? 8 : 4;
+}
+
+// The untuned configuration of an index box.  Rows per thread: 4 re-read the
+// fewest halo rows, 2 and 1 give a small or thin box enough workgroups.  Two planes
+// ahead where there are few rows to load a plane (not in the residuals, which
+// hold f too).  Non-temporal stores where the result would not stay in the
+// 256 MB cache anyway.  Every configuration was timed over cubes of 48..512
+// cells; this rule is within 10 % of the best.  Against the fixed shape before
+// it (2 rows in FP64, 4 in FP32, cached stores, 16 planes or more; us):
+//                    64^3          160^3         512^3
+//   7-point FP64     7.1 ->  5.6   14.4 -> 13.5  431 -> 387
+//   27-point FP64   10.0 ->  5.5   20.0 -> 20.2  450 -> 388
+//   27-point FP32   13.1 ->  6.0   16.1 -> 14.0  244 -> 217
+//   2 residuals F64 19.2 -> 11.4   36.8 -> 36.2  878 -> 764
+static ZCfg default_cfg(int mode, int dtype, const Box3& ibox)
+{
+    ZCfg c;
+    c.ry = box_nz(ibox) >= 16 && zblocks(ibox, 4, 16) >= 768 ? 4 : (zblocks(ibox, 2, 4) >= 512 ? 2 : 1);
+    c.pf = c.ry == 4 || mode >= ZM_RESIDUAL ? 1 : 2;
+    c.nt = box_size(ibox) * (long)dtype_size(dtype) >= 96L << 20 ? 1 : 0;
+    c.tz = 0;
+    return c;
+}
 
 // Tuned configurations per (operator kind, mode, dtype, index-box shape).
 struct TuneKey {
@@ -686,7 +728,7 @@ static ZCfg lookup_cfg(int kind, int mode, int dtype, const Box3& ib)
         auto it = g_tune->find(tune_key(kind, mode, dtype, ib));
         if (it != g_tune->end()) { return it->second; }
     }
-    return default_cfg(dtype);
+    return default_cfg(mode, dtype, ib);
 }
 
 static void store_cfg(const TuneKey& k, const ZCfg& c)
@@ -707,13 +749,7 @@ static ZPlan zplan(const Box3& ibox, const ZCfg& c)
     const int nx = (int)box_nx(ibox), ny = (int)box_ny(ibox), nz = (int)box_nz(ibox);
     p.ntx = (nx + 63) / 64;
     p.nty = (ny + 4 * c.ry - 1) / (4 * c.ry);
-    int tz = nz;
-    if (c.tz > 0) {
-        tz = std::min(c.tz, nz);
-    } else {
-        // enough blocks to fill 256 CUs several times over, but long z runs
-        while (tz > 16 && (long)p.ntx * p.nty * ((nz + tz - 1) / tz) < 4096) { tz = (tz + 1) / 2; }
-    }
+    const int tz = std::min(c.tz > 0 ? c.tz : auto_tz(ibox, c.ry), nz);
     p.tz = tz;
     p.ntz = (nz + tz - 1) / tz;
     p.blocks = (unsigned)((long)p.ntx * p.nty * p.ntz);
@@ -1017,8 +1053,8 @@ static int autotune_t(const pm_stencil* st, const pm_stencil* st2, int mode, con
                       ZCfg* best, float* best_ms, hipStream_t s)
 {
     const size_t ns = (size_t)box_size(sb), ni = (size_t)box_size(ib);
-    // the most blocks any candidate launches: one row per thread, 16 planes
-    const size_t maxb = (size_t)((box_nx(ib) + 63) / 64) * (size_t)((box_ny(ib) + 3) / 4) * (size_t)((box_nz(ib) + 15) / 16);
+    // the most blocks any candidate launches: one row per thread, 4 planes (the automatic chunk's least)
+    const size_t maxb = (size_t)((box_nx(ib) + 63) / 64) * (size_t)((box_ny(ib) + 3) / 4) * (size_t)((box_nz(ib) + 3) / 4);
     T *src = nullptr, *dst = nullptr, *dst2 = nullptr, *f = nullptr, *part = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = PM_OK;
@@ -1056,7 +1092,7 @@ static int autotune_t(const pm_stencil* st, const pm_stencil* st2, int mode, con
     const int nz = (int)box_nz(ib);
     const int tzs[6] = {0, 16, 32, 64, 128, 256};
     float bms = 1e30f;
-    ZCfg bc = default_cfg(dtype_of<T>::value);
+    ZCfg bc = default_cfg(mode, dtype_of<T>::value, ib);
     for (int ry : kRY)
         for (int pf = 1; pf <= 2; pf++)
             for (int nt = 0; nt <= 1; nt++)
