@@ -120,6 +120,42 @@ def test_generic_zmarch_random_stencils(dtype):
         assert out.tobytes() == ref.tobytes(), trial
 
 
+@pytest.mark.parametrize("ntap", [1, 3, 4, 5, 32, 33, 70])
+@pytest.mark.parametrize("dtype", [pa.PM_F64, pa.PM_F32])
+def test_wide_and_ratio_stencils_vs_oracle(dtype, ntap):
+    """Stencils of the generic kernel (offsets to +-3, refinement ratios and
+    shifts): tap groups of four and their remainder, lists in the arguments and
+    in the handle, fewer planes than a thread takes and one more, rows that are
+    not wave multiples, two components, replace and accumulate; bitwise."""
+    rng = np.random.default_rng(77 + ntap)
+    npdt = np.float64 if dtype == pa.PM_F64 else np.float32
+    pool = np.array([(x, y, z) for z in range(-3, 4) for y in range(-3, 4) for x in range(-3, 4)], dtype=np.int32)
+    for trial, (n, sr, dr, ds) in enumerate([((37, 5, 1), 1, 1, 0), ((65, 9, 3), 1, 1, 0), ((129, 4, 4), 1, 1, 0),
+                                             ((31, 17, 5), 2, 1, 0), ((20, 11, 9), 1, 2, 1)]):
+        o = pool[rng.permutation(len(pool))[:ntap]].copy()
+        o[0] = (3, -3, 2)  # wide whatever was drawn
+        c = rng.uniform(-2, 2, size=ntap).astype(npdt)
+        st = pa.Stencil(c, o, dtype, 3, (sr,) * 3, (dr,) * 3, (ds,) * 3)
+        assert st.kind() == 0
+        lo = np.array([-2, 1, 3])
+        hi = lo + np.array(n) - 1
+        slo, shi = lo * sr - 3, hi * sr + 4
+        dlo, dhi = lo * dr + ds - 1, hi * dr + ds + 1
+        replace, scale = trial % 2 == 0, [1.0, -0.75][trial % 2]
+        say("wide", dtype, ntap, "trial", trial)
+        ns, nd = util.box_size(slo, shi), util.box_size(dlo, dhi)
+        src = util.uniform(900 + trial, 0, 2 * ns).astype(npdt)
+        dst0 = util.uniform(900 + trial, 1, 2 * nd).astype(npdt)
+        ref = dst0.copy()
+        for q in range(2):
+            r = ref[q * nd:(q + 1) * nd].copy()
+            util.oracle_apply(c, o, src[q * ns:(q + 1) * ns].copy(), slo, shi, r, dlo, dhi, lo, hi, replace, scale,
+                              (sr,) * 3, (dr,) * 3, (ds,) * 3)
+            ref[q * nd:(q + 1) * nd] = r
+        out = apply_gpu(st, src, slo, shi, dst0.copy(), dlo, dhi, lo, hi, replace, scale, ncomp=2)
+        assert out.tobytes() == ref.tobytes(), trial
+
+
 @pytest.mark.parametrize("name", ["Laplacian", "Laplacian_27"])
 def test_kernel_families_agree(name):
     """The 7/27-point z-march, the generic z-march and the per-cell kernel
