@@ -32,7 +32,7 @@ struct pm_fas {
     };
     std::vector<Level> lv;
     double* d_part = nullptr;  // per-block maxima of the residual norm
-    double* d_norm = nullptr;
+    double* h_norm = nullptr;  // pinned host scalar the norm kernel writes
     size_t cap_part = 0;
     size_t bytes = 0;
 };
@@ -768,10 +768,10 @@ static int fas_resnorm(pm_fas* M, void* u, const void* f, double* out, hipStream
                            (const double*)u, (const double*)f, fas_coefs(Lv.dx), M->d_part, res_out);
     }
     hipLaunchKernelGGL(k_fas_max, dim3(1), dim3(1024), 0, s, (const double*)M->d_part, (long)bpb * D.nboxes,
-                       M->d_norm);
+                       M->h_norm);
     PM_CHECK_LAUNCH();
-    PM_CHECK_HIP(hipMemcpyAsync(out, M->d_norm, sizeof(double), hipMemcpyDeviceToHost, s));
     PM_CHECK_HIP(hipStreamSynchronize(s));
+    *out = *M->h_norm;
     return PM_OK;
 }
 
@@ -806,7 +806,7 @@ int pm_fas_destroy(pm_fas* M)
         pm_layout_destroy(L.layout);
     }
     hipFree(M->d_part);
-    hipFree(M->d_norm);
+    if (M->h_norm) { hipHostFree(M->h_norm); }
     delete M;
     return PM_OK;
 }
@@ -866,7 +866,12 @@ int pm_fas_create(pm_fas** out, const pm_layout* fine, int num_levels, double dx
         if (l == 0) { maxpart = (size_t)fas_blocks((long)e0 / D.nboxes) * D.nboxes; }
     }
     if (rc == PM_OK) { rc = fas_alloc(M, (void**)&M->d_part, 8 * std::max<size_t>(maxpart, 1)); }
-    if (rc == PM_OK) { rc = fas_alloc(M, (void**)&M->d_norm, 64); }
+    if (rc == PM_OK && hipHostMalloc((void**)&M->h_norm, 64, hipHostMallocDefault) != hipSuccess) {
+        set_error("pm_fas_create: pinned host allocation failed");
+        M->h_norm = nullptr;
+        rc = PM_ERR_NOMEM;
+    }
+    M->bytes += 64;
     if (rc != PM_OK) {
         pm_fas_destroy(M);
         return rc;

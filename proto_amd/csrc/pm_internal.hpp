@@ -72,6 +72,27 @@ int level_restrict_nb(const pm_layout* F, const pm_layout* C, int dtype, const v
 int level_sweep_restrict(const pm_layout* F, const pm_layout* C, int dtype, const void* phi_in,
                          const int in_ghost[3], void* phi_out, const int out_ghost[3], const void* rhs,
                          const int rhs_ghost[3], double dx, void* resc, const int resc_ghost[3], hipStream_t stream);
+// Whether the sweeps choose their kernel themselves (pm_level_sweep_form 0) (pm_level.hip).
+bool level_sweep_auto();
+// Levels that live in cache (pm_block.hip).  level_block_ok: periodic levels
+// covering their domain, box-aligned with their coarse level C, of boxes of 6 or
+// more and an even number of cells a side, small enough for it to pay.
+// level_block_down: two sweeps of phi (ghost 1; the zero guess with zero_in)
+// into tmp (no ghosts) and their residual restricted into the coarse
+// right-hand side crhs (no ghosts).  level_block_up: two sweeps of tmp + the
+// constant prolongation of cphi (ghost 1) into phi (ghost 1), or added to the
+// FP64 solution acc of phi's layout.  rhs has no ghosts.
+bool level_block_ok(const pm_layout* L, const pm_layout* C, int dtype);
+int level_block_down(const pm_layout* L, const pm_layout* C, int dtype, const void* phi, int zero_in, void* tmp,
+                     const void* rhs, double dx, void* crhs, hipStream_t stream);
+int level_block_up(const pm_layout* L, const pm_layout* C, int dtype, const void* tmp, const void* cphi, void* phi,
+                   double* acc, const void* rhs, double dx, hipStream_t stream);
+// A V-cycle from level lv[0] to the coarsest lv.back() in one launch, in place
+// on phi (ghost 1): one-box periodic levels of even sizes, each half the one
+// before, the first of at most 4096 cells, at most four.  PM_ERR_UNSUPPORTED
+// (without a message) otherwise.
+int level_bottom(const std::vector<const pm_layout*>& lv, const std::vector<double>& dx, int dtype, int pre, int post,
+                 int bottom, void* phi, const void* rhs, bool zero_in, hipStream_t stream);
 // Kernel family (0 generic, 7, 27), dtype and coefficients of a stencil (pm_stencil.hip).
 int stencil_info(const pm_stencil* st, int* kind, int* dtype, std::vector<double>* coefs);
 

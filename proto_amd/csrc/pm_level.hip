@@ -2583,6 +2583,8 @@ int level_gsrb_sweep_in(const pm_layout* L, int dtype, const void* phi_in, const
 #undef PM_SWEEP_MODES
 #undef PM_SWEEP_LAUNCH
 
+bool level_sweep_auto() { return g_sweep_form == 0; }
+
 bool levels_box_aligned(const pm_layout* F, const pm_layout* C) { return box_aligned(F, C); }
 
 int level_gsrb_small(const pm_layout* L, int dtype, void* phi, const int phi_ghost[3], const void* rhs,

@@ -31,7 +31,7 @@ struct pm_mg {
         void* tmp32 = nullptr;
     };
     std::vector<Level> lv;
-    void* d_norm = nullptr;  // device scalar for norms
+    double* h_norm = nullptr;  // pinned host scalar the norm kernels write (no copy to read it back)
     size_t bytes = 0;
     int g1[3] = {1, 1, 1};
     int g0[3] = {0, 0, 0};
@@ -88,7 +88,7 @@ static void mg_free(pm_mg* mg)
         hipFree(l.tmp32);
         pm_layout_destroy(l.layout);
     }
-    hipFree(mg->d_norm);
+    if (mg->h_norm) { hipHostFree(mg->h_norm); }
     if (mg->gexec) { hipGraphExecDestroy(mg->gexec); }
     if (mg->graph) { hipGraphDestroy(mg->graph); }
 }
@@ -186,10 +186,32 @@ static int vcycle(pm_mg* mg, int l, int dtype, void* phi, const void* rhs, hipSt
     int pre = mg->opt.pre, post = mg->opt.post, bottom = mg->opt.bottom;
     if (mg->opt.relax == 1) { pre = post = 2 * mg->dim; bottom = 10; }
     const int zin = zero_in ? 1 : 0;
+    const bool small = mg->opt.relax == 0 && mg->opt.fused && mg->dim == 3 && mg->opt.interp == 0 && level_sweep_auto();
+    if (small) {
+        // the last levels, down to the coarsest, in one launch
+        std::vector<const pm_layout*> lays;
+        std::vector<double> dxs;
+        for (int k = l; k <= mg->nlev; k++) {
+            lays.push_back(mg->lv[k].layout);
+            dxs.push_back(mg->lv[k].dx);
+        }
+        const int rc = level_bottom(lays, dxs, dtype, pre, post, bottom, phi, rhs, zero_in, s);
+        if (rc != PM_ERR_UNSUPPORTED) { return rc; }
+    }
     if (l < mg->nlev) {
         auto& C = mg->lv[l + 1];
         void* cphi = f32 ? C.phi32 : C.phi;
         void* crhs = f32 ? C.rhs32 : C.rhs;
+        if (small && pre == 2 && post == 2 && level_block_ok(L.layout, C.layout, dtype)) {
+            // a level that lives in cache: both pre-smoothing sweeps and the
+            // residual restriction in one pass (phi -> tmp), the prolongation
+            // and both post-smoothing sweeps in another (tmp -> phi)
+            MG_TRY(level_block_down(L.layout, C.layout, dtype, phi, zin, tmp, rhs, L.dx, crhs, s));
+            MG_TRY(vcycle(mg, l + 1, dtype, cphi, crhs, s, true));
+            MG_TRY(level_block_up(L.layout, C.layout, dtype, tmp, cphi, phi, acc64, rhs, L.dx, s));
+            if (acc64) { *folded = true; }
+            return PM_OK;
+        }
         // coarseResidual (51-73): exchange, residual, AvgDown, copy to the coarse
         // layout; where the level qualifies it is computed by the last
         // pre-smoothing sweep, else the halo is read from the neighbouring boxes
@@ -222,8 +244,8 @@ static int vcycle(pm_mg* mg, int l, int dtype, void* phi, const void* rhs, hipSt
 
 static int read_norm(pm_mg* mg, double* out, hipStream_t s)
 {
-    PM_CHECK_HIP(hipMemcpyAsync(out, mg->d_norm, sizeof(double), hipMemcpyDeviceToHost, s));
     PM_CHECK_HIP(hipStreamSynchronize(s));
+    *out = *mg->h_norm;
     return PM_OK;
 }
 
@@ -233,10 +255,10 @@ static int read_norm(pm_mg* mg, double* out, hipStream_t s)
 static int resnorm(pm_mg* mg, void* phi, const void* rhs, double* out, hipStream_t s)
 {
     auto& L = mg->lv[0];
-    const int rc = level_resnorm_nb(L.layout, PM_F64, phi, mg->g1, rhs, mg->g0, L.dx, mg->d_norm, 0, s);
+    const int rc = level_resnorm_nb(L.layout, PM_F64, phi, mg->g1, rhs, mg->g0, L.dx, mg->h_norm, 0, s);
     if (rc == PM_ERR_UNSUPPORTED) {
         MG_TRY(pm_level_exchange(L.layout, PM_F64, phi, mg->g1, 1, s));
-        MG_TRY(pm_level_resnorm(L.layout, PM_F64, phi, mg->g1, rhs, mg->g0, L.dx, mg->d_norm, 0, s));
+        MG_TRY(pm_level_resnorm(L.layout, PM_F64, phi, mg->g1, rhs, mg->g0, L.dx, mg->h_norm, 0, s));
     } else if (rc != PM_OK) {
         return rc;
     }
@@ -248,11 +270,11 @@ static int residual32(pm_mg* mg, void* phi, const void* rhs, hipStream_t s)
 {
     auto& L = mg->lv[0];
     const int rc = level_residual_nb(L.layout, PM_F64, phi, mg->g1, rhs, mg->g0, L.dx, PM_F32, L.rhs32, mg->g0,
-                                     mg->d_norm, s);
+                                     mg->h_norm, s);
     if (rc == PM_ERR_UNSUPPORTED) {
         MG_TRY(pm_level_exchange(L.layout, PM_F64, phi, mg->g1, 1, s));
         MG_TRY(pm_level_residual(L.layout, PM_F64, phi, mg->g1, rhs, mg->g0, L.dx, PM_F32, L.rhs32, mg->g0,
-                                 mg->d_norm, s));
+                                 mg->h_norm, s));
     } else if (rc != PM_OK) {
         return rc;
     }
@@ -412,7 +434,12 @@ int pm_mg_create(pm_mg** out, const pm_layout* fine, int nlevels, double dx, con
             if (need_tmp && rc == PM_OK) { rc = dalloc(mg, &L.tmp32, 4 * e0); }
         }
     }
-    if (rc == PM_OK) { rc = dalloc(mg, &mg->d_norm, 64); }
+    if (rc == PM_OK && hipHostMalloc((void**)&mg->h_norm, 64, hipHostMallocDefault) != hipSuccess) {
+        set_error("multigrid: pinned host allocation failed");
+        mg->h_norm = nullptr;
+        rc = PM_ERR_NOMEM;
+    }
+    mg->bytes += 64;
     if (rc != PM_OK) {
         mg_free(mg);
         delete mg;

@@ -281,6 +281,38 @@ def test_row_and_tile_sweeps_same_solve(precision, n, nlev):
         assert p1.tobytes() == p0.tobytes(), form
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n,bs,nlev", [(8, 8, 2), (16, 16, 1), (20, 20, 1), (24, 24, 2), (24, 12, 1), (36, 12, 1),
+                                       (36, 18, 1), (40, 8, 2), (44, 22, 1), (64, 32, 3), (96, 48, 4), (128, 32, 4)])
+def test_block_levels_same_solve(precision, n, bs, nlev):
+    """Levels that live in cache (two sweeps and the transfer in one pass, the
+    last levels in one launch): tiles that divide the boxes and ragged ones, one
+    box and several in an order of their own, bottoms of one to three levels, the
+    largest FP32 level; the same histories and bits as the tile sweeps."""
+    lows = [(x, y, z) for z in range(0, n, bs) for y in range(0, n, bs) for x in range(0, n, bs)]
+    L = Layout(n, bs, [lows[i] for i in np.random.default_rng(n).permutation(len(lows))])
+    rhs = util.gaussian_rhs(n, 5, 8)
+    rd = dev(L.pack(rhs, 0))
+    res = {}
+    try:
+        for form in (1, 0):
+            pa.call("pm_level_sweep_form", form)
+            opt = pa.MgOptions()
+            pa.lib().pm_mg_default_options(ctypes.byref(opt))
+            opt.precision, opt.inner, opt.max_iter, opt.tol = precision, 2, 4, 1e-14
+            mg = ctypes.c_void_p()
+            pa.call("pm_mg_create", ctypes.byref(mg), L.h, nlev, 1.0 / n, ctypes.byref(opt))
+            phi, hist, it = zeros(len(lows) * (bs + 2) ** 3), np.zeros(5), ctypes.c_int()
+            say("block levels", n, bs, nlev, "form", form)
+            pa.lib().pm_mg_solve(mg, vp(phi), vp(rd), hist.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
+                                 ctypes.byref(it), None)
+            res[form] = (it.value, hist.tobytes(), host(phi).tobytes())
+            pa.call("pm_mg_destroy", mg)
+    finally:
+        pa.call("pm_level_sweep_form", 0)
+    assert res[0] == res[1]
+
+
 def test_gsrb_sweep_unsupported_layouts():
     hole = Layout(32, 16, lows=[(0, 0, 0), (16, 0, 0)])
     buf = zeros(2 * 18 ** 3)
