@@ -27,12 +27,13 @@
 #include <thread>
 #include <vector>
 
+#include "pm_block.hpp"
 #include "pm_internal.hpp"
 
 namespace pm {
 
 constexpr int SR = 8;    // rows per sweep tile
-constexpr int SZC = 32;  // planes per sweep tile
+constexpr int SZC = 32;  // most planes per sweep tile
 constexpr int SCELLS = 2048;  // cells per item of the pointwise kernels
 
 struct SLevel {
@@ -344,6 +345,82 @@ __global__ __launch_bounds__(256) void k_srv_small(const SLevel* __restrict__ lv
     for (int i = threadIdx.x; i < N; i += 256) { L.phi[i] = u[i]; }
 }
 
+// Two sweeps of a tile of a request's level in one pass (pm_block.hpp; the level
+// is one periodic box, so every neighbouring box is the box itself): IN 0 / 1
+// from phi or the zero guess into tmp, with the residual restricted into the
+// next level's rhs; IN 2 from tmp + the prolongation into phi, or (OUT 1) added to
+// the request's FP64 solution.  Item: tile corner a, b, c, tile size packed in x0.
+// 24 requests of 32^3 .. 128^3 in one burst: the solves 11.4 -> 8.1 ms with these
+// passes below the finest levels, k_srv_bottom and the shorter sweep tiles.
+template<int IN, int OUT>
+__global__ __launch_bounds__(kBlkThreads) void k_srv_block(const SLevel* __restrict__ lv, const SItem* __restrict__ items)
+{
+    constexpr int RES = IN == 2 ? 0 : 1;
+    __shared__ float u[kBlkPhi], f[kBlkRhs];
+    __shared__ BlockBases s;
+    if (threadIdx.x < 27) { s.in[threadIdx.x] = s.rhs[threadIdx.x] = s.crs[threadIdx.x] = 0; }
+    const SItem it = items[blockIdx.x];
+    const SLevel L = lv[it.lev], C = lv[it.lev + 1];
+    BlockTile<float> B;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        B.n[d] = L.n;
+        B.t[d] = (it.x0 >> (8 * d)) & 255;
+    }
+    B.t0[0] = it.a;
+    B.t0[1] = it.b;
+    B.t0[2] = it.c;
+    B.par = 0;
+    B.in = IN == 2 ? L.tmp : L.phi;
+    B.rhs = L.rhs;
+    B.crs = C.phi;
+    B.out = IN == 2 ? L.phi : L.tmp;
+    B.acc = L.acc;
+    B.crhs = C.rhs;
+    B.ix = B.rx = B.ox = L.n;
+    B.ixy = B.rxy = B.oxy = L.n * L.n;
+    B.cx = B.qx = C.n;
+    B.cxy = B.qxy = C.n * C.n;
+    B.c0 = B.r0 = L.c0;
+    B.c1 = B.r1 = L.c1;
+    B.lam = L.lam;
+    B.avg = 0.125f;
+    __syncthreads();
+    block_two_sweeps<float, IN, OUT, RES>(B, s, u, f);
+}
+
+// The levels of a request from it.lev (n^3 <= 4096) down to its coarsest, it.a of
+// them, in one workgroup from the zero guess (pm_block.hpp).
+__global__ __launch_bounds__(kBotThreads) void k_srv_bottom(const SLevel* __restrict__ lv, const SItem* __restrict__ items,
+                                                            int pre, int post, int bottom)
+{
+    __shared__ float u[kBotStore], f[kBotStore];
+    __shared__ BottomArgs<float> A;
+    const SItem it = items[blockIdx.x];
+    if ((int)threadIdx.x < it.a) {
+        const SLevel L = lv[it.lev + threadIdx.x];
+        BottomLevel<float>& B = A.lv[threadIdx.x];
+        B.n[0] = B.n[1] = B.n[2] = L.n;
+        B.c0 = B.r0 = L.c0;
+        B.c1 = B.r1 = L.c1;
+        B.lam = L.lam;
+    }
+    if (threadIdx.x == 0) {
+        A.nl = it.a;
+        A.par = 0;
+        A.pre = pre;
+        A.post = post;
+        A.bottom = bottom;
+        A.avg = 0.125f;
+    }
+    const SLevel T = lv[it.lev];
+    const int N = T.n * T.n * T.n;
+    for (int i = threadIdx.x; i < N; i += kBotThreads) { f[i] = T.rhs[i]; }
+    __syncthreads();
+    bottom_cycle<float>(A, u, f, true);
+    for (int i = threadIdx.x; i < N; i += kBotThreads) { T.phi[i] = u[i]; }
+}
+
 // Coarse right-hand side = AvgDown(rhs + sum_j c_j phi(p + o_j)) of the fine
 // level (LevelMultigrid.cpp:51-73 order), and, with zero_phi, coarse phi = 0
 // (otherwise the coarse level's first sweep takes the zero guess as its input).
@@ -589,7 +666,7 @@ struct HeldRun {
 };
 
 struct Launch {
-    int kind;  // 0 sweep, 1 restrict, 2 prolong, 3 correct, 4 residual, 5 small-level relaxation
+    int kind;  // 0 sweep, 1 restrict, 2 prolong, 3 correct, 4 residual, 5 small-level relaxation, 6 block pass, 7 bottom
     int off, count, dir;
     int in;    // sweeps: staged input (k_srv_gsrb IN), 3 = IN 0 with OUT 1; restrict / residual: 1 = write the zero guess
     size_t lds;  // sweeps: dynamic LDS of the largest tile
@@ -782,12 +859,12 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
         L.count = (int)items.size() - L.off;
         if (L.count == 0) { S->plan.pop_back(); }
     };
-    auto sweep_items = [&](int levidx, int m) {
+    auto sweep_items = [&](int levidx, int m, int zc) {
         const int r = sweep_rows(m), w = sweep_cols(m);
-        for (int z0 = 0; z0 < m; z0 += SZC)
+        for (int z0 = 0; z0 < m; z0 += zc)
             for (int y0 = 0; y0 < m; y0 += r)
                 for (int x0 = 0; x0 < m; x0 += w) {
-                    items.push_back(SItem{levidx, y0, z0, std::min(m, z0 + SZC), x0, std::min(m, x0 + w)});
+                    items.push_back(SItem{levidx, y0, z0, std::min(m, z0 + zc), x0, std::min(m, x0 + w)});
                 }
         Launch& L = S->plan.back();
         L.lds = std::max(L.lds, sweep_lds(m));
@@ -803,6 +880,57 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
     // levels below the finest of at most SMALL_CELLS cells relax in one launch
     // each (k_srv_small), all requests' such levels of one depth together
     auto small = [&](const Active& a, int d) { return d > 0 && (long)a.ns[d] * a.ns[d] * a.ns[d] <= SMALL_CELLS; };
+    // From 64^3 cells in flight on, the forms below.  Fewer keep one launch per
+    // operator and 32-plane tiles, though these are the slower ones there too (a
+    // lone 32^3 request: 0.7 ms against more than 1): test_alone_equals_in_mix
+    // holds that a request arriving 1 ms after a 32^3 one still meets it in flight.
+    long cells0 = 0;
+    for (const Active& a : act) { cells0 += (long)a.ns[0] * a.ns[0] * a.ns[0]; }
+    const bool many = cells0 > 64L * 64 * 64;
+    // The bottom of a request's hierarchy from depth d on in one launch: a level
+    // below the finest of at most 4096 cells, even sizes down to the coarsest.
+    auto bottom = [&](const Active& a, int d) {
+        if (!many || !zero_in || !fold_prolong || d >= (int)a.ns.size() || !small(a, d)) { return false; }
+        bool ok = (int)a.ns.size() - d <= kBotLevels;
+        for (size_t l = d; l < a.ns.size(); l++) { ok = ok && a.ns[l] % 2 == 0; }
+        return ok;
+    };
+    auto below_bottom = [&](const Active& a, int d) { return d > 0 && bottom(a, d - 1); };
+    // Depths whose levels together live in cache run two sweeps and the transfer in
+    // one pass (pm_block.hpp); at most 128^3 cells over all requests, as the
+    // driver's FP32 levels.  The sweeps of the other depths cut their boxes into
+    // chunks of 32, 16 or 8 planes for about 2048 tiles: their time is the z walk
+    // (1.5 us a plane) until the chip is full.
+    std::vector<char> blk(maxd + 1, 0);
+    std::vector<int> zcs(maxd + 1, SZC);
+    for (int d = 0; d <= maxd; d++) {
+        long cells = 0, cols = 0;
+        const bool ok = many && pre == 2 && post == 2 && zero_in;
+        for (const Active& a : act) {
+            if (a.fresh || d >= (int)a.ns.size() || bottom(a, d) || below_bottom(a, d)) { continue; }
+            const long m = a.ns[d];
+            cells += m * m * m;
+            cols += ((m + sweep_cols((int)m) - 1) / sweep_cols((int)m)) * ((m + SR - 1) / SR) * m;
+        }
+        blk[d] = ok && cells <= 128L * 128 * 128;
+        while (many && zcs[d] > 8 && cols / zcs[d] < 2048) { zcs[d] /= 2; }
+    }
+    auto block = [&](const Active& a, int d) {
+        return blk[d] && d < (int)a.ns.size() - 1 && a.ns[d] >= 6 && a.ns[d] % 2 == 0 && !bottom(a, d) && !below_bottom(a, d);
+    };
+    auto block_items = [&](int levidx, int m) {
+        const int n[3] = {m, m, m};
+        int nt[3], tl[3];
+        block_tiles(n, 1, nt, tl);
+        for (int z = 0; z < m; z += tl[2])
+            for (int y = 0; y < m; y += tl[1])
+                for (int x = 0; x < m; x += tl[0]) {
+                    const int w[3] = {std::min(tl[0], m - x), std::min(tl[1], m - y), std::min(tl[2], m - z)};
+                    items.push_back(SItem{levidx, x, y, z, w[0] | w[1] << 8 | w[2] << 16, 0});
+                }
+    };
+    // levels that no other form takes
+    auto plain = [&](const Active& a, int d) { return !block(a, d) && !bottom(a, d) && !below_bottom(a, d); };
     // `inner` V-cycles of every non-fresh request (fresh ones only get their first
     // residual): the first takes the zero initial guess on every level, the later
     // ones start level 0 from the previous cycle's correction; only the last
@@ -813,11 +941,23 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
     for (int d = 0; d <= maxd; d++) {
         // level 0 of a later cycle reads its correction; coarser levels start from zero
         const bool zin = zero_in && (d > 0 || cyc == 0);
+        begin(7, 0);
+        for (size_t r = 0; r < act.size(); r++) {
+            const Active& a = act[r];
+            if (a.fresh || !bottom(a, d) || below_bottom(a, d)) { continue; }
+            items.push_back(SItem{lev0[r] + d, (int)a.ns.size() - d, 0, 0, 0, 0});
+        }
+        end();
+        begin(6, 0, zin ? 1 : 0);
+        for (size_t r = 0; r < act.size(); r++) {
+            if (!act[r].fresh && block(act[r], d)) { block_items(lev0[r] + d, act[r].ns[d]); }
+        }
+        end();
         begin(5, 0, zin ? 1 : 0);
         for (size_t r = 0; r < act.size(); r++) {
             const Active& a = act[r];
             const int bd = (int)a.ns.size() - 1;
-            if (a.fresh || d > bd || !small(a, d)) { continue; }
+            if (a.fresh || d > bd || !small(a, d) || !plain(a, d)) { continue; }
             const int cnt = d < bd ? pre : bot;
             if (cnt > 0) { items.push_back(SItem{lev0[r] + d, cnt, 0, 0, 0, 0}); }
         }
@@ -828,15 +968,15 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
             for (size_t r = 0; r < act.size(); r++) {
                 const Active& a = act[r];
                 const int bd = (int)a.ns.size() - 1;
-                if (a.fresh || d > bd || small(a, d)) { continue; }
-                if ((d < bd && sw < pre) || (d == bd && sw < bot)) { sweep_items(lev0[r] + d, a.ns[d]); }
+                if (a.fresh || d > bd || small(a, d) || !plain(a, d)) { continue; }
+                if ((d < bd && sw < pre) || (d == bd && sw < bot)) { sweep_items(lev0[r] + d, a.ns[d], zcs[d]); }
             }
             end();
         }
         begin(1, 0, zero_in ? 0 : 1);
         for (size_t r = 0; r < act.size(); r++) {
             const Active& a = act[r];
-            if (a.fresh || d >= (int)a.ns.size() - 1) { continue; }
+            if (a.fresh || d >= (int)a.ns.size() - 1 || !plain(a, d)) { continue; }
             const long c = (long)a.ns[d + 1] * a.ns[d + 1] * a.ns[d + 1];
             push_cells(items, lev0[r] + d, c);
         }
@@ -847,16 +987,22 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
             begin(2, 0);
             for (size_t r = 0; r < act.size(); r++) {
                 const Active& a = act[r];
-                if (a.fresh || d >= (int)a.ns.size() - 1) { continue; }
+                if (a.fresh || d >= (int)a.ns.size() - 1 || !plain(a, d)) { continue; }
                 push_cells(items, lev0[r] + d, (long)a.ns[d] * a.ns[d] * a.ns[d]);
             }
             end();
         }
+        // the last pass of level 0 adds e into the FP64 solution
+        begin(6, 1, last_cycle && d == 0 ? 3 : 2);
+        for (size_t r = 0; r < act.size(); r++) {
+            if (!act[r].fresh && block(act[r], d)) { block_items(lev0[r] + d, act[r].ns[d]); }
+        }
+        end();
         if (post > 0) {
             begin(5, 0, fold_prolong ? 2 : 0);
             for (size_t r = 0; r < act.size(); r++) {
                 const Active& a = act[r];
-                if (a.fresh || d >= (int)a.ns.size() - 1 || !small(a, d)) { continue; }
+                if (a.fresh || d >= (int)a.ns.size() - 1 || !small(a, d) || !plain(a, d)) { continue; }
                 items.push_back(SItem{lev0[r] + d, post, 0, 0, 0, 0});
             }
             end();
@@ -867,8 +1013,8 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
             begin(0, sw & 1, last_cycle && d == 0 && sw == post - 1 && in == 0 ? 3 : in);
             for (size_t r = 0; r < act.size(); r++) {
                 const Active& a = act[r];
-                if (a.fresh || d >= (int)a.ns.size() - 1 || small(a, d)) { continue; }
-                sweep_items(lev0[r] + d, a.ns[d]);
+                if (a.fresh || d >= (int)a.ns.size() - 1 || small(a, d) || !plain(a, d)) { continue; }
+                sweep_items(lev0[r] + d, a.ns[d], zcs[d]);
             }
             end();
         }
@@ -946,6 +1092,21 @@ int run_plan(pm_server* S, int nact, hipStream_t s)
             } else {
                 hipLaunchKernelGGL(k_srv_small<2>, dim3(L.count), dim3(256), 0, s, (const SLevel*)S->d_lv, it);
             }
+            break;
+        case 6:
+            if (L.in == 0) {
+                hipLaunchKernelGGL((k_srv_block<0, 0>), dim3(L.count), dim3(kBlkThreads), 0, s, (const SLevel*)S->d_lv, it);
+            } else if (L.in == 1) {
+                hipLaunchKernelGGL((k_srv_block<1, 0>), dim3(L.count), dim3(kBlkThreads), 0, s, (const SLevel*)S->d_lv, it);
+            } else if (L.in == 2) {
+                hipLaunchKernelGGL((k_srv_block<2, 0>), dim3(L.count), dim3(kBlkThreads), 0, s, (const SLevel*)S->d_lv, it);
+            } else {
+                hipLaunchKernelGGL((k_srv_block<2, 1>), dim3(L.count), dim3(kBlkThreads), 0, s, (const SLevel*)S->d_lv, it);
+            }
+            break;
+        case 7:
+            hipLaunchKernelGGL(k_srv_bottom, dim3(L.count), dim3(kBotThreads), 0, s, (const SLevel*)S->d_lv, it,
+                               S->opt.pre, S->opt.post, S->opt.bottom);
             break;
         case 2:
             hipLaunchKernelGGL(k_srv_prolong, dim3(L.count), dim3(256), 0, s, (const SLevel*)S->d_lv, it);
