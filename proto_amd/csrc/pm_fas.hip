@@ -18,6 +18,7 @@
 #include <cstring>
 #include <vector>
 
+#include "pm_block.hpp"
 #include "pm_layout.hpp"
 
 struct pm_fas {
@@ -149,13 +150,17 @@ __global__ __launch_bounds__(256) void k_fas_op_z(LayoutDev L, const double* __r
     __shared__ double sm[4][FZ_NE];
     __shared__ double red[16];
     __shared__ int s_nb[NB ? 27 : 1], s_dz[NB ? 18 : 1], s_dc[IN == 2 ? 18 : 1];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int b = blockIdx.y;
     const int nx = L.bs[0], ny = L.bs[1], nz = L.bs[2];
-    const int nyt = (ny + FZ_TY - 1) / FZ_TY;
-    const int y0 = (int)(blockIdx.x % nyt) * FZ_TY;
+    // boxes 32 wide: two row groups a wave (32 lanes each), tiles of 32 x 16, instead
+    // of half the lanes idle (128^3 in 32^3 boxes: 22.6 -> 19.1 us a relaxation)
+    const bool narrow = nx <= 32;
+    const int TY = narrow ? 2 * FZ_TY : FZ_TY;
+    const int nyt = (ny + TY - 1) / TY;
+    const int y0 = (int)(blockIdx.x % nyt) * TY;
     const int z0 = (int)(blockIdx.x / nyt) * zc, z1 = min(z0 + zc, nz);
-    const int LX = nx + 4, NE = (FZ_TY + 4) * LX;
+    const int LX = nx + 4, NE = (TY + 4) * LX;
     const long X = nx + 4, XY = X * (ny + 4), vol = XY * (nz + 4);
     const double* ub = u + (long)b * vol;
     const long nv = (long)nx * ny * nz;
@@ -266,7 +271,8 @@ __global__ __launch_bounds__(256) void k_fas_op_z(LayoutDev L, const double* __r
             if (e < NE) { pl[e] = v; }
         }
     };
-    const int x = lane;
+    const int x = narrow ? lane & 31 : lane;
+    const int w = narrow ? 2 * (tid >> 6) + (lane >> 5) : tid >> 6;  // row group: rows y0 + w RY ..
     const bool xok = x < nx;
     const int xc = xok ? x : 0;  // idle lanes read column 0 (results never stored)
     double zw[5][RY];             // own cells of planes zo-2 .. zo+2
@@ -482,6 +488,324 @@ __global__ __launch_bounds__(256) void k_fas_relax_small(LayoutDev L, double* __
     }
 }
 
+// fas_L at element i of an LDS array: neighbours at the given offsets (x, y, z:
+// -2, -1, +1, +2 cells).
+__device__ __forceinline__ double fas_L_lds(const double* u, int i, const int (&x)[4], const int (&y)[4],
+                                            const int (&z)[4], double uc, const FasC& c)
+{
+    double acc = 0;
+    auto dim = [&](const int (&o)[4]) {
+        const double m2 = u[i + o[0]], m1 = u[i + o[1]], p1 = u[i + o[2]], p2 = u[i + o[3]];
+        double fr = 0;
+        fr = fr + c.a[0] * m1;
+        fr = fr + c.a[1] * uc;
+        fr = fr + c.a[2] * p1;
+        fr = fr + c.a[3] * p2;
+        double fl = 0;
+        fl = fl + c.a[0] * m2;
+        fl = fl + c.a[1] * m1;
+        fl = fl + c.a[2] * uc;
+        fl = fl + c.a[3] * p1;
+        acc = acc + c.dp * fr;
+        acc = acc + c.dm * fl;
+    };
+    dim(x);
+    dim(y);
+    dim(z);
+    double o = 0;
+    o = o + acc;
+    return o * -1.0;
+}
+
+// Two Jacobi relaxations of a tile of at most 16 x 8 x 8 cells in one pass, for
+// levels that live in cache: the tile and a 4-cell halo, read from the
+// neighbouring boxes' valid cells, are staged in LDS at once (72 KB with f, two
+// workgroups a CU); the first sweep covers the tile grown by 2 cells, each thread
+// holding its new values until every old one is read.  IN 2: the staged input is
+// u + the constant prolongation of the coarse correction (crse0 - crseState) * -1,
+// formed here from both (k_fas_delta is not run), as k_fas_op_z stages it.
+// The arithmetic is fas_L's, so the bits are k_fas_relax's.  Levels of up to
+// 128^3 cells are bound by the z walk of k_fas_op_z (12 planes of latency and a
+// barrier each a launch): 64^3 and 32^3 levels 13 and 11 us a sweep there, 11 us
+// for two here.  Register count: the first sweep's cells one at a time, 53.
+constexpr int kFasH = 4;
+constexpr int kFasU = (kBlkX + 2 * kFasH) * (kBlkY + 2 * kFasH) * (kBlkZ + 2 * kFasH);
+constexpr int kFasF = (kBlkX + 4) * (kBlkY + 4) * (kBlkZ + 4);
+
+template<int IN>
+__global__ __launch_bounds__(kBlkThreads, 4) void k_fas_block(LayoutDev L, const double* __restrict__ u,
+                                                          const double* __restrict__ f, double* __restrict__ out, FasC c,
+                                                          LayoutDev C, const double* __restrict__ cu,
+                                                          const double* __restrict__ cu0, int ntx, int nty, int ntz, int tx,
+                                                          int ty, int tz)
+{
+    __shared__ double su[kFasU], sf[kFasF];
+    __shared__ int bu[27], bf[27], bc[27], bc0[27];
+    constexpr int H = kFasH;
+    const int tid = threadIdx.x;
+    const int tiles = ntx * nty * ntz, at_box = blockIdx.x / tiles, t = blockIdx.x - at_box * tiles;
+    const int px = at_box % L.nb[0], pr = at_box / L.nb[0], py = pr % L.nb[1], pz = pr / L.nb[1];
+    const int nx = L.bs[0], ny = L.bs[1], nz = L.bs[2];
+    const int X = nx + 4, XY = X * (ny + 4), vol = XY * (nz + 4), nv = nx * ny * nz;
+    const int CX0 = C.bs[0], CXY0 = CX0 * C.bs[1], CX = CX0 + 4, CXY = CX * (C.bs[1] + 4);
+    auto wrap = [](int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); };
+    if (tid < 27) {
+        const int x = wrap(px + tid % 3 - 1, L.nb[0]), y = wrap(py + (tid / 3) % 3 - 1, L.nb[1]),
+                  z = wrap(pz + tid / 9 - 1, L.nb[2]);
+        const int o = L.table[x + L.nb[0] * (y + L.nb[1] * z)];
+        bu[tid] = o * vol + 2 + 2 * X + 2 * XY;
+        bf[tid] = o * nv;
+        if (IN == 2) {
+            const int q[3] = {(x * nx) >> 1, (y * ny) >> 1, (z * nz) >> 1};
+            const int cb[3] = {small_div(q[0], C.bs[0]), small_div(q[1], C.bs[1]), small_div(q[2], C.bs[2])};
+            const int oc = C.table[cb[0] + C.nb[0] * (cb[1] + C.nb[1] * cb[2])];
+            const int r[3] = {q[0] - cb[0] * C.bs[0], q[1] - cb[1] * C.bs[1], q[2] - cb[2] * C.bs[2]};
+            bc[tid] = oc * CXY * (C.bs[2] + 4) + (r[0] + 2) + CX * (r[1] + 2) + CXY * (r[2] + 2);
+            bc0[tid] = oc * CXY0 * C.bs[2] + r[0] + CX0 * r[1] + CXY0 * r[2];
+        }
+    }
+    const int b = L.table[at_box];
+    const int ax = t % ntx, ar = t / ntx, ay = ar % nty, az = ar / nty;
+    const int x0 = ax * tx, y0 = ay * ty, z0 = az * tz;
+    tx = min(tx, nx - x0);
+    ty = min(ty, ny - y0);
+    tz = min(tz, nz - z0);
+    __syncthreads();
+    // staging: 32 lanes a row, 16 rows at a time, U rows in flight a lane
+    const int col = tid & 31, rg = tid >> 5;
+    constexpr int G = kBlkThreads / 32, U = 8;
+    auto side = [](int v, int n) { return v < 0 ? 0 : (v >= n ? 2 : 1); };
+    auto stage = [&](auto&& load, double* dst, int h) {
+        const int w = tx + 2 * h, hy = ty + 2 * h, hz = tz + 2 * h, rows = hy * hz;
+        const int x = x0 - h + min(col, w - 1), kx = side(x, nx), xl = x - (kx - 1) * nx;
+        const int dq = small_div(G, hy), dm = G - dq * hy;
+        int zz = small_div(rg, hy), yy = rg - zz * hy;
+        for (int r0 = rg; r0 < rows; r0 += G * U) {
+            double v[U];
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                const int y = y0 - h + yy, z = z0 - h + min(zz, hz - 1), ky = side(y, ny), kz = side(z, nz);
+                v[i] = load(kx + 3 * ky + 9 * kz, xl, y - (ky - 1) * ny, z - (kz - 1) * nz);
+                yy += dm;
+                zz += dq;
+                if (yy >= hy) {
+                    yy -= hy;
+                    zz++;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                const int r = r0 + G * i;
+                if (r < rows && col < w) { dst[col + __mul24(w, r)] = v[i]; }
+            }
+        }
+    };
+    stage(
+        [&](int k, int x, int y, int z) -> double {
+            const double v = u[bu[k] + x + __mul24(X, y) + __mul24(XY, z)];
+            if constexpr (IN == 2) {
+                const int xc = x >> 1, yc = y >> 1, zc = z >> 1;
+                const double d = cu0[bc0[k] + xc + __mul24(CX0, yc) + __mul24(CXY0, zc)] -
+                                 cu[bc[k] + xc + __mul24(CX, yc) + __mul24(CXY, zc)];
+                const double zero = 0;
+                return v + (zero + d * -1.0);
+            } else {
+                return v;
+            }
+        },
+        su, H);
+    stage([&](int k, int x, int y, int z) -> double { return f[bf[k] + x + __mul24(nx, y) + __mul24(nx * ny, z)]; }, sf, 2);
+    __syncthreads();
+    const int W = tx + 2 * H, P = W * (ty + 2 * H), WF = tx + 4, PF = WF * (ty + 4);
+    const int ox[4] = {-2, -1, 1, 2}, oy[4] = {-2 * W, -W, W, 2 * W}, oz[4] = {-2 * P, -P, P, 2 * P};
+    auto cell = [&](int x, int y, int z) {  // tile coordinates: the relaxed value
+        const int i = (x + H) + __mul24(W, y + H) + __mul24(P, z + H);
+        const double uc = su[i];
+        double res = fas_L_lds(su, i, ox, oy, oz, uc, c);
+        res = res + sf[(x + 2) + __mul24(WF, y + 2) + __mul24(PF, z + 2)];
+        return uc + c.mlam * res;
+    };
+    // first sweep: the tile grown by 2
+    {
+        const int w = tx + 4, h = ty + 4, n = w * h * (tz + 4);
+        constexpr int M = (kFasF + kBlkThreads - 1) / kBlkThreads;
+        double v[M];
+        int li[M];
+#pragma unroll
+        for (int i = 0; i < M; i++) {
+            const int e = min(tid + kBlkThreads * i, n - 1), r = small_div(e, w), z = small_div(r, h), x = e - r * w, y = r - z * h;
+            v[i] = cell(x - 2, y - 2, z - 2);
+            li[i] = (x - 2 + H) + __mul24(W, y - 2 + H) + __mul24(P, z - 2 + H);
+            // computed here, not sunk into the conditional store below with all its operands live
+            asm volatile("" : "+v"(v[i]));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < M; i++) {
+            if (tid + kBlkThreads * i < n) { su[li[i]] = v[i]; }
+        }
+        __syncthreads();
+    }
+    // second sweep: the tile, straight out
+    const int lx = tid & 15, lr = tid >> 4;
+    double* ob = out + (long)b * vol + 2 + 2 * X + 2 * XY;
+#pragma unroll
+    for (int i = 0; i < kBlkY * kBlkZ * 16 / kBlkThreads; i++) {
+        const int r = lr + (kBlkThreads / 16) * i, z = small_div(r, ty), y = r - z * ty;
+        if (lx < tx && z < tz) { ob[(x0 + lx) + X * (y0 + y) + XY * (z0 + z)] = cell(lx, y, z); }
+    }
+}
+
+// The levels from a one-box periodic level of at most 2048 cells down to the
+// coarsest in one workgroup, everything in LDS (40 KB): relaxations, averageDown,
+// crseForce, the correction and its prolongation, term by term as the kernels of
+// the larger levels.  Bound by LDS latency: each of its up to 22 relaxations and
+// transfers was one to three launches of 5 to 47 us.  A larger top level is better
+// spread over workgroups by k_fas_block: 16^3 here 112 us a cycle, there 90; 12^3
+// here 30 us less.
+constexpr int kFasBotCells = 2048;
+constexpr int kFasBotStore = kFasBotCells + kFasBotCells / 8 + kFasBotCells / 64 + kFasBotCells / 512;
+
+struct FasBottom {
+    int nl;
+    int n[kBotLevels][3];
+    FasC c[kBotLevels];
+};
+
+__global__ __launch_bounds__(kBotThreads) void k_fas_bottom(FasBottom args, double* __restrict__ ug,
+                                                            const double* __restrict__ fg)
+{
+    __shared__ FasBottom A;  // indexed by level: in LDS, not in a private copy
+    if (threadIdx.x == 0) { A = args; }
+    __syncthreads();
+    __shared__ double su[kFasBotStore], sf[kFasBotStore], s0[kFasBotStore - kFasBotCells];
+    constexpr int M = kFasBotCells / kBotThreads;
+    const int tid = threadIdx.x;
+    auto fold = [](int v, int n) {  // -2 .. n + 1 into 0 .. n - 1, n at least 2
+        return v < 0 ? v + n : (v >= n ? v - n : v);
+    };
+    // offsets of the neighbours of cell (x, y, z)
+    auto offsets = [&](const int (&n)[3], int x, int y, int z, int (&ox)[4], int (&oy)[4], int (&oz)[4]) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int d = k < 2 ? k - 2 : k - 1;
+            ox[k] = fold(x + d, n[0]) - x;
+            oy[k] = n[0] * (fold(y + d, n[1]) - y);
+            oz[k] = n[0] * n[1] * (fold(z + d, n[2]) - z);
+        }
+    };
+    auto relax = [&](int l, double* u, const double* f, int nsw) {
+        const int n[3] = {A.n[l][0], A.n[l][1], A.n[l][2]}, N = n[0] * n[1] * n[2];
+        const FasC c = A.c[l];
+        // neighbour offsets of this thread's cells, two signed 16-bit ones a register
+        int pk[M][6];
+#pragma unroll
+        for (int i = 0; i < M; i++) {
+            const int e = min(tid + kBotThreads * i, N - 1), r = small_div(e, n[0]), z = small_div(r, n[1]);
+            int o[3][4];
+            offsets(n, e - r * n[0], r - z * n[1], z, o[0], o[1], o[2]);
+#pragma unroll
+            for (int k = 0; k < 6; k++) { pk[i][k] = (o[k / 2][2 * (k & 1)] & 0xffff) | (o[k / 2][2 * (k & 1) + 1] << 16); }
+        }
+        for (int sw = 0; sw < nsw; sw++) {
+            double v[M];
+#pragma unroll
+            for (int i = 0; i < M; i++) {
+                const int e = tid + kBotThreads * i;
+                v[i] = 0;
+                if (e < N) {
+                    const double uc = u[e];
+                    int o[3][4];
+#pragma unroll
+                    for (int k = 0; k < 6; k++) {
+                        asm volatile("" : "+v"(pk[i][k]));  // unpacked here, not held unpacked over the sweeps
+                        o[k / 2][2 * (k & 1)] = (short)pk[i][k];
+                        o[k / 2][2 * (k & 1) + 1] = pk[i][k] >> 16;
+                    }
+                    double res = fas_L_lds(u, e, o[0], o[1], o[2], uc, c);
+                    res = res + f[e];
+                    v[i] = uc + c.mlam * res;
+                }
+                asm volatile("" : "+v"(v[i]));  // computed before the barrier
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < M; i++) {
+                const int e = tid + kBotThreads * i;
+                if (e < N) { u[e] = v[i]; }
+            }
+            __syncthreads();
+        }
+    };
+    const int nx = A.n[0][0], ny = A.n[0][1], nz = A.n[0][2], X = nx + 4, XY = X * (ny + 4);
+    auto at = [&](int e) {
+        const int r = small_div(e, nx), z = small_div(r, ny);
+        return (e - r * nx + 2) + X * (r - z * ny + 2) + XY * (z + 2);
+    };
+    for (int e = tid; e < nx * ny * nz; e += kBotThreads) {
+        su[e] = ug[at(e)];
+        sf[e] = fg[e];
+    }
+    __syncthreads();
+    int off = 0, c0 = 0;  // of the level in su and sf; of its coarse level in s0
+    for (int l = 0;; l++) {
+        const int n[3] = {A.n[l][0], A.n[l][1], A.n[l][2]}, N = n[0] * n[1] * n[2];
+        double* u = su + off;
+        double* f = sf + off;
+        const bool last = l == A.nl - 1;
+        relax(l, u, f, last ? 10 : 6);
+        if (last) { break; }
+        // averageDown of the state, then crseForce = AvgDown(L(u) + f) - L_c(crseState)
+        const int m[3] = {n[0] >> 1, n[1] >> 1, n[2] >> 1}, NC = N / 8;
+        double* uc = u + N;
+        double* u0 = s0 + c0;
+        const bool own = tid < NC;  // at most 256 coarse cells
+        const int r = small_div(own ? tid : 0, m[0]), Z = small_div(r, m[1]), Xc = (own ? tid : 0) - r * m[0], Y = r - Z * m[1];
+        double avg = 0, force = 0;
+        if (own) {
+#pragma unroll 1
+            for (int k = 0; k < 8; k++) {
+                const int x = 2 * Xc + (k & 1), y = 2 * Y + ((k >> 1) & 1), z = 2 * Z + (k >> 2);
+                const int e = x + n[0] * (y + n[1] * z);
+                avg = avg + 0.125 * u[e];
+                int ox[4], oy[4], oz[4];
+                offsets(n, x, y, z, ox, oy, oz);
+                double res = fas_L_lds(u, e, ox, oy, oz, u[e], A.c[l]);
+                res = res + f[e];
+                force = force + 0.125 * res;
+            }
+            uc[tid] = avg;
+            u0[tid] = avg;
+        }
+        __syncthreads();
+        if (own) {
+            int ox[4], oy[4], oz[4];
+            offsets(m, Xc, Y, Z, ox, oy, oz);
+            f[N + tid] = force - fas_L_lds(uc, tid, ox, oy, oz, uc[tid], A.c[l + 1]);
+        }
+        __syncthreads();
+        off += N;
+        c0 += NC;
+    }
+    for (int l = A.nl - 2; l >= 0; l--) {
+        const int n[3] = {A.n[l][0], A.n[l][1], A.n[l][2]}, N = n[0] * n[1] * n[2], mx = n[0] >> 1, my = n[1] >> 1;
+        const double* uc = su + off;
+        c0 -= N / 8;
+        const double* u0 = s0 + c0;
+        off -= N;
+        double* u = su + off;
+        for (int e = tid; e < N; e += kBotThreads) {
+            const int r = small_div(e, n[0]), z = small_div(r, n[1]), x = e - r * n[0], y = r - z * n[1];
+            const int k = (x >> 1) + mx * ((y >> 1) + my * (z >> 1));
+            const double d = u0[k] - uc[k], zero = 0;
+            u[e] = u[e] + (zero + d * -1.0);
+        }
+        __syncthreads();
+        relax(l, u, sf + off, 6);
+    }
+    for (int e = tid; e < nx * ny * nz; e += kBotThreads) { ug[at(e)] = su[e]; }
+}
+
 // per-block max |L(u) + f|
 __global__ __launch_bounds__(256) void k_fas_resnorm(LayoutDev L, G3 gu, G3 gf, const double* __restrict__ u,
                                                      const double* __restrict__ f, FasC c, double* __restrict__ part,
@@ -629,12 +953,16 @@ static bool fz_nb(const pm_layout* L)
     return gvol(D, g3(G2)) * L->nboxes < (1L << 31);
 }
 
-// its grid: 16-row tiles x z chunks (halved while fewer than 2048 workgroups) x boxes
+// its grid: 8-row tiles (16 rows of 32-wide boxes) x z chunks (halved while fewer than
+// 2048 workgroups) x boxes
 static dim3 fz_grid(const LayoutDev& D, int* zc)
 {
-    const int nyt = (D.bs[1] + FZ_TY - 1) / FZ_TY;
+    const int ty = D.bs[0] <= 32 ? 2 * FZ_TY : FZ_TY, nyt = (D.bs[1] + ty - 1) / ty;
+    auto blocks = [&](int z) { return (long)nyt * ((D.bs[2] + z - 1) / z) * D.nboxes; };
     int z = D.bs[2];
-    while (z > 8 && (long)nyt * ((D.bs[2] + z - 1) / z) * D.nboxes < 2048) { z = (z + 1) / 2; }
+    while (z > 8 && blocks(z) < 2048) { z = (z + 1) / 2; }
+    // 128^3 cells: 4 planes 9.1 ms a solve, 8 planes 9.8; 192^3: 13.4 against 12.6
+    if (z > 4 && z <= 8 && blocks(z) < 1024) { z = (z + 1) / 2; }
     *zc = z;
     return dim3((unsigned)(nyt * ((D.bs[2] + z - 1) / z)), (unsigned)D.nboxes);
 }
@@ -700,12 +1028,98 @@ static int fas_relax(pm_fas* M, int l, void* u, const void* f, int n, hipStream_
     return PM_OK;
 }
 
-static int fas_vcycle(pm_fas* M, int l, void* u, const void* f, hipStream_t s)
+// A V-cycle from level l on in one launch (k_fas_bottom): one-box periodic levels
+// of even sizes, the first of at most kFasBotCells cells, at most four.
+static bool fas_bottom_ok(const pm_fas* M, int l)
 {
-    if (l == M->nlev) { return fas_relax(M, l, u, f, 10, s); }
+    if (M->nlev - l + 1 > kBotLevels) { return false; }
+    for (int k = l; k <= M->nlev; k++) {
+        const pm_layout* L = M->lv[k].layout;
+        if (L->nboxes != 1 || L->nb[0] * L->nb[1] * L->nb[2] != 1 ||
+            (long)L->bs[0] * L->bs[1] * L->bs[2] > (kFasBotCells >> (3 * (k - l)))) {
+            return false;
+        }
+        for (int d = 0; d < 3; d++) {
+            if (!L->periodic[d] || L->bs[d] % 2) { return false; }
+        }
+    }
+    return true;
+}
+
+static int fas_bottom(pm_fas* M, int l, void* u, const void* f, hipStream_t s)
+{
+    FasBottom A;
+    A.nl = M->nlev - l + 1;
+    for (int k = 0; k < A.nl; k++) {
+        for (int d = 0; d < 3; d++) { A.n[k][d] = M->lv[l + k].layout->bs[d]; }
+        A.c[k] = fas_coefs(M->lv[l + k].dx);
+    }
+    hipLaunchKernelGGL(k_fas_bottom, dim3(1), dim3(kBotThreads), 0, s, A, (double*)u, (const double*)f);
+    PM_CHECK_LAUNCH();
+    return PM_OK;
+}
+
+// Levels whose relaxations go two a launch (k_fas_block): periodic, every box
+// present, boxes of 4 or more and an even number of cells a side, box-aligned with
+// the coarse level, small enough for the recomputed halo (1.9 times the cells) to
+// pay.
+static bool fas_block_ok(const pm_fas* M, int l)
+{
+    if (l == M->nlev) { return false; }
+    const pm_layout* L = M->lv[l].layout;
+    if (L->nboxes != L->nb[0] * L->nb[1] * L->nb[2] || !levels_box_aligned(L, M->lv[l + 1].layout)) { return false; }
+    long cells = 1;
+    for (int d = 0; d < 3; d++) {
+        if (!L->periodic[d] || L->bs[d] < 4 || L->bs[d] % 2) { return false; }
+        cells *= L->domain[d];
+    }
+    // us of a solve to 1e-6 with every level of up to 64^3 / 96^3 / 128^3 cells so:
+    // 32^3 boxes, 128^3 cells (17 cycles) 12261 / 12254 / 13983, 48^3 boxes, 96^3
+    // cells 5687 / 5983 / -, but 16^3 boxes (whose other form is an exchange and a
+    // per-cell kernel a sweep), 128^3 cells 16842 / 16818 / 14625
+    const long side = fz_ok(ldev(L)) ? 72 : 160;
+    return cells <= side * side * side;
+}
+
+// Six relaxations of level l from buffer `from` into buffer `to` (three launches);
+// correct: fineCorrect is still to be applied to `from`.
+static int fas_relax6(pm_fas* M, int l, void* from, void* to, const void* f, bool correct, hipStream_t s)
+{
+    const pm_layout* L = M->lv[l].layout;
+    const pm_layout* CL = M->lv[l + 1].layout;
+    const FasC c = fas_coefs(M->lv[l].dx);
+    int nt[3], tl[3];
+    block_tiles(L->bs, L->nboxes, nt, tl);
+    const unsigned blocks = (unsigned)(nt[0] * nt[1] * nt[2] * L->nboxes);
+    for (int i = 0; i < 3; i++) {
+        const double* in = (const double*)(i & 1 ? to : from);
+        double* out = (double*)(i & 1 ? from : to);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlkThreads), 0, s, ldev(L), in, (const double*)f, out, c, ldev(CL),
+                               (const double*)M->lv[l + 1].phi, (const double*)M->lv[l + 1].phi0, nt[0], nt[1], nt[2], tl[0],
+                               tl[1], tl[2]);
+        };
+        if (i == 0 && correct) { go(k_fas_block<2>); } else { go(k_fas_block<0>); }
+    }
+    PM_CHECK_LAUNCH();
+    return PM_OK;
+}
+
+static int fas_vcycle(pm_fas* M, int l, void* state, const void* f, hipStream_t s)
+{
+    if (fas_bottom_ok(M, l)) { return fas_bottom(M, l, state, f, s); }
+    if (l == M->nlev) { return fas_relax(M, l, state, f, 10, s); }
     auto& F = M->lv[l];
     auto& C = M->lv[l + 1];
-    FAS_TRY(fas_relax(M, l, u, f, 6, s));
+    // two relaxations a launch: the smoothed state lies in the scratch buffer, from
+    // where the post relaxations' odd count of launches brings it back
+    const bool block = fas_block_ok(M, l);
+    void* u = block ? F.tmp : state;
+    if (block) {
+        FAS_TRY(fas_relax6(M, l, state, u, f, false, s));
+    } else {
+        FAS_TRY(fas_relax(M, l, u, f, 6, s));
+    }
     const LayoutDev DF = ldev(F.layout), DC = ldev(C.layout);
     // crseForce from the z-marching operator kernel where the fine level reads
     // its neighbours (then u needs no exchange: averageDown reads valid cells)
@@ -732,6 +1146,7 @@ static int fas_vcycle(pm_fas* M, int l, void* u, const void* f, hipStream_t s)
     }
     PM_CHECK_LAUNCH();
     FAS_TRY(fas_vcycle(M, l + 1, C.phi, C.f, s));
+    if (block) { return fas_relax6(M, l, u, state, f, true, s); }
     hipLaunchKernelGGL(k_fas_delta, grid, dim3(256), 0, s, DC, g3(G2), g3(G0), (const double*)C.phi, (double*)C.phi0);
     PM_CHECK_LAUNCH();
     // fineCorrect (u += I(delta)) folded into the first post relaxation

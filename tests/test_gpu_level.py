@@ -539,3 +539,20 @@ def test_fas_vs_oracle(n, bs, levels):
     assert it == oit
     assert hist.tobytes() == ohist[:oit + 1].tobytes()
     assert phi.tobytes() == ophi.tobytes()
+
+
+@pytest.mark.parametrize("n,bs,levels", [(8, 8, 1), (12, 12, 2), (16, 16, 2), (20, 20, 2), (24, 24, 3), (24, 12, 2),
+                                         (36, 18, 2), (40, 8, 3), (44, 22, 2), (48, 24, 3), (64, 32, 4), (80, 16, 4)])
+def test_fas_block_levels_vs_oracle(n, bs, levels):
+    """Relaxations two a launch (tiles that divide the boxes and ragged ones, boxes
+    wide enough for the z-marching residual and not, one box and several), the
+    correction formed in the first of them, and the last levels in one launch,
+    from one level to three."""
+    say("fas block levels", n, bs, levels)
+    force = util.gaussian_rhs(n, 5, 17)
+    it, hist, phi = _fas(n, bs, levels, force, maxiter=3)
+    ophi, ohist = np.zeros(n ** 3), np.zeros(5)
+    oit = util.oracle().orc_fas_solve(n, levels, util.ptr(force), util.ptr(ophi), 3, 1e-10, util.ptr(ohist))
+    assert it == oit
+    assert hist.tobytes() == ohist[:oit + 1].tobytes()
+    assert phi.tobytes() == ophi.tobytes()
