@@ -19,13 +19,6 @@
 
 namespace pm {
 
-// a / d for 0 <= a < 2^20 and 0 < d: the quotient's distance from the next
-// integer is at least 0.5 / d, far above the reciprocal's error.
-__device__ inline int small_div(int a, int d)
-{
-    return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)d));
-}
-
 // Tiles of at most 16 x 8 x 8 cells; 512 threads (two waves a SIMD) hide the
 // LDS latency of a colour pass.  LDS: 8424 + 6144 values, 57 KB in FP32 (two
 // workgroups a CU), 114 KB in FP64 (one).

@@ -212,6 +212,13 @@ __device__ __forceinline__ double lane_shift(double edge, double v)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
+// a / d for 0 <= a < 2^20 and 0 < d: the quotient's distance from the next
+// integer is at least 0.5 / d, far above the reciprocal's error.
+__device__ inline int small_div(int a, int d)
+{
+    return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+}
+
 // XCD-aware block remap: MI355X dispatches workgroup i to XCD (i mod 8); this
 // hands each XCD a contiguous run of logical tiles so that tiles sharing halo
 // rows share that XCD's L2.

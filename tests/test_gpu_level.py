@@ -556,3 +556,30 @@ def test_fas_block_levels_vs_oracle(n, bs, levels):
     assert it == oit
     assert hist.tobytes() == ohist[:oit + 1].tobytes()
     assert phi.tobytes() == ophi.tobytes()
+
+
+@pytest.mark.parametrize("dt", [pa.PM_F64, pa.PM_F32])
+@pytest.mark.parametrize("bs,ghost,ncomp", [(4, (1, 1, 1), 1), (4, (4, 4, 4), 5), (6, (2, 0, 3), 4), (8, (0, 3, 1), 3),
+                                            (10, (3, 1, 2), 8), (4, (5, 5, 5), 2)])
+def test_exchange_components_and_ghosts(dt, bs, ghost, ncomp):
+    """Every ghost cell of every component is its periodic image, every valid cell
+    kept: components in groups of four and the rest, ghost widths that differ by
+    direction, as wide as a box and wider (the general kernel), an order of boxes
+    of its own."""
+    n = 3 * bs
+    lows = [(x, y, z) for z in range(0, n, bs) for y in range(0, n, bs) for x in range(0, n, bs)]
+    lows = [lows[i] for i in np.random.default_rng(bs).permutation(len(lows))]
+    L = Layout(n, bs, lows)
+    t = np.float64 if dt == pa.PM_F64 else np.float32
+    glob = util.uniform(41, 0, ncomp * n ** 3).astype(t).reshape(ncomp, n, n, n)
+    gx, gy, gz = ghost
+    want = np.zeros((len(lows), ncomp, bs + 2 * gz, bs + 2 * gy, bs + 2 * gx), dtype=t)
+    data = np.full_like(want, -7)
+    for b, (x, y, z) in enumerate(lows):
+        i = [np.arange(lo - g, lo + bs + g) % n for lo, g in ((z, gz), (y, gy), (x, gx))]
+        want[b] = glob[:, i[0]][:, :, i[1]][:, :, :, i[2]]
+        data[b, :, gz:gz + bs, gy:gy + bs, gx:gx + bs] = glob[:, z:z + bs, y:y + bs, x:x + bs]
+    d = dev(data.reshape(-1))
+    say("exchange", dt, bs, ghost, ncomp)
+    pa.call("pm_level_exchange", L.h, dt, vp(d), pa.i3(ghost), ncomp, None)
+    assert host(d).tobytes() == want.tobytes()
