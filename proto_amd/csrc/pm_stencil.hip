@@ -604,7 +604,9 @@ __global__ __launch_bounds__(256) void k_zgen(ZArgs<T> a)
     finish();
 }
 
-// The one-block second stage of k_zgen's reductions (fixed strided split and tree).
+// The one-block second stage of k_zgen's reductions (fixed strided split and tree
+// for a count of partials).  As many threads as partials, whole waves, at most 1024:
+// a 256^2 apply + absMax 9.2 -> 7.5 us against always 1024.
 template<typename T>
 __global__ __launch_bounds__(1024) void k_finish_op(int op, const T* __restrict__ partials, int nb, T* out,
                                                     int combine)
@@ -753,25 +755,26 @@ static long zblocks(const Box3& ibox, int ry, int tz)
 // Planes per workgroup where the configuration leaves them open: long runs
 // stage less halo (a run of tz stages tz + 2 planes), short ones reach all 256
 // CUs and end sooner (a plane takes a few hundred ns of load latency and
-// barriers).  16 where that still gives three workgroups a CU, then 8, then 4;
-// more than 16 only to keep the count of workgroups (and their partials)
-// bounded.
+// barriers).  16 from about 460^3 cells on, 8 while that leaves four workgroups a
+// CU, else 4; more than 16 only to keep the count
+// of workgroups (and their partials) bounded.
 static int auto_tz(const Box3& ibox, int ry)
 {
-    if (zblocks(ibox, ry, 16) >= 768) {
+    if (zblocks(ibox, ry, 16) >= 6000) {
         int tz = 16;
         while (zblocks(ibox, ry, tz) > 16384 && tz < box_nz(ibox)) { tz *= 2; }
         return tz;
     }
-    return zblocks(ibox, ry, 8) >= 768 ? 8 : 4;
+    return zblocks(ibox, ry, 8) >= 1024 ? 8 : 4;
 }
 
 // The untuned configuration of an index box.  Rows per thread: 4 re-read the
 // fewest halo rows, 2 and 1 give a small or thin box enough workgroups.  Two planes
 // ahead where there are few rows to load a plane (not in the residuals, which
-// hold f too).  Non-temporal stores where the result would not stay in the
-// 256 MB cache anyway.  Every configuration was timed over cubes of 48..512
-// cells; this rule is within 10 % of the best.  Against the fixed shape before
+// hold f too).  Non-temporal stores where the result would not stay in cache
+// anyway (200^3 FP64, three arrays in turn: 38.8 -> 21.5 us).  Every configuration
+// was timed over cubes of 48..512 cells and boxes such as 137 x 209 x 283; this
+// rule is within 10 % of the best of nearly all.  Against the fixed shape before
 // it (2 rows in FP64, 4 in FP32, cached stores, 16 planes or more; us):
 //                    64^3          160^3         512^3
 //   7-point FP64     7.1 ->  5.6   14.4 -> 13.5  431 -> 387
@@ -781,9 +784,10 @@ static int auto_tz(const Box3& ibox, int ry)
 static ZCfg default_cfg(int mode, int dtype, const Box3& ibox)
 {
     ZCfg c;
-    c.ry = box_nz(ibox) >= 16 && zblocks(ibox, 4, 16) >= 768 ? 4 : (zblocks(ibox, 2, 4) >= 512 ? 2 : 1);
+    c.ry = (box_nz(ibox) >= 16 || dtype == PM_F32) && zblocks(ibox, 4, 16) >= 768 ? 4
+                                                                                   : (zblocks(ibox, 2, 4) >= 512 ? 2 : 1);
     c.pf = c.ry == 4 || mode >= ZM_RESIDUAL ? 1 : 2;
-    c.nt = box_size(ibox) * (long)dtype_size(dtype) >= 96L << 20 ? 1 : 0;
+    c.nt = box_size(ibox) * (long)dtype_size(dtype) >= 32L << 20 ? 1 : 0;
     c.tz = 0;
     return c;
 }
@@ -1360,7 +1364,7 @@ int pm_stencil_apply_reduce(const pm_stencil* st, const void* src, const pm_box*
             int r2 = replace ? launch_zgen<T, ZM_REPLACE>(st, a, ib, cfg, s, true)
                              : launch_zgen<T, ZM_ACCUM>(st, a, ib, cfg, s, true);
             if (r2) { return r2; }
-            hipLaunchKernelGGL(k_finish_op<T>, dim3(1), dim3(1024), 0, s, op, (const T*)ws, (int)nb, (T*)out_dev,
+            hipLaunchKernelGGL(k_finish_op<T>, dim3(1), dim3(std::min(1024u, (nb + 63) & ~63u)), 0, s, op, (const T*)ws, (int)nb, (T*)out_dev,
                                combine);
             PM_CHECK_LAUNCH();
             return PM_OK;
