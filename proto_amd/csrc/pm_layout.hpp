@@ -10,6 +10,7 @@ struct pm_layout {
     int dim;
     int domain[3], bs[3], periodic[3], nb[3];
     int nboxes;
+    bool x_pairs;  // boxes 2 i and 2 i + 1 along x both there and one after the other in layout order
     std::vector<int> lows;
     int* d_lows;
     int* d_table;

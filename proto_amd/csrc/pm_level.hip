@@ -469,11 +469,11 @@ __global__ __launch_bounds__(256) void k_gsrb_fused(LayoutDev L, G3 gin, G3 gout
 
 // ------------------------------------------------------------ row-register sweep
 
-// One full red-black sweep of a periodic level of boxes 64 cells wide that
-// covers its domain, out of place, in one pass, the rows held in registers.
-// A workgroup is one wave per box column of the domain (at most 8): lane l of
-// wave w holds column 64 w + l, so the workgroup holds whole rows of the
-// domain.  It owns rows [Y0, Y0 + RY) of one box row and planes [Z0, Z1) of
+// One full red-black sweep of a periodic level of boxes 64 cells wide (BW 64; or
+// 32, two boxes to a wave, stored one after another) that covers its domain, out
+// of place, in one pass, the rows held in registers.  A workgroup is one wave per
+// 64 columns of the domain (at most 8): lane l of wave w holds column 64 w + l,
+// so the workgroup holds whole rows of the domain.  It owns rows [Y0, Y0 + RY) of one box row and planes [Z0, Z1) of
 // one box layer; each thread keeps its column of rows [Y0 - 2, Y0 + RY + 2)
 // of the planes in use in registers and walks z.  Step k: the red cells of
 // plane k + 1 over the tile rows and one halo row on each side (the values
@@ -488,7 +488,7 @@ __global__ __launch_bounds__(256) void k_gsrb_fused(LayoutDev L, G3 gin, G3 gout
 // out are template arguments).  Arithmetic, order and colouring are k_gsrb's;
 // IN (0 phi, 1 zero guess, 2 phi + the constant prolongation of a coarse level
 // with one ghost layer) and OUT as k_gsrb_fused.
-template<typename T, int RY, int IN, int OUT, int NT, int GP, int GR, int GO, int PF>
+template<typename T, int RY, int IN, int OUT, int NT, int GP, int GR, int GO, int PF, int BW>
 __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restrict__ pin, T* __restrict__ pout,
                                                    const T* __restrict__ rhs, Lap<T> c, T lambda, int zc,
                                                    double* __restrict__ pacc, LayoutDev C,
@@ -496,7 +496,8 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
 {
     constexpr int NR = RY + 4;  // phi rows held: Y0 - 2 .. Y0 + RY + 1
     constexpr int NQ = RY + 2;  // rhs rows: Y0 - 1 .. Y0 + RY
-    constexpr long XP = 64 + 2 * GP, XR = 64 + 2 * GR, XO = 64 + 2 * GO;
+    constexpr int NB = 64 / BW;  // boxes a wave holds
+    constexpr long XP = BW + 2 * GP, XR = BW + 2 * GR, XO = BW + 2 * GO;
     using TO = typename std::conditional<OUT == 1, double, T>::type;  // what the output array holds
     __shared__ T eo[2][8][2][NQ];   // old values of a plane's edge lanes (0, 63), rows Y0 - 1 .. Y0 + RY
     __shared__ T er[2][8][2][RY];   // red-updated edge values, rows Y0 .. Y0 + RY - 1
@@ -505,7 +506,7 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
     // kernel argument would copy it to private memory)
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int nw = L.nb[0], nb1 = L.nb[1], nb2 = L.nb[2];
+    const int nb0 = L.nb[0], nw = nb0 / NB, nb1 = L.nb[1], nb2 = L.nb[2];
     const int bs1 = L.bs[1], bs2 = L.bs[2], dom1 = L.domain[1];
     const int wl = w == 0 ? nw - 1 : w - 1, wr = w == nw - 1 ? 0 : w + 1;
     const int nyt = dom1 / RY;
@@ -519,7 +520,7 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
     const int* table = L.table;
     auto box_at = [&](int ys, int zs) __attribute__((always_inline)) {
         const int yb = (by + ys + nb1) % nb1, zb = (bz + zs + nb2) % nb2;
-        return table[w + nw * (yb + nb1 * zb)];
+        return table[w * NB + nb0 * (yb + nb1 * zb)];
     };
     // boxes of the three row classes for the planes below / in / above the box layer
     const int tm = box_at(ytop, -1), t0 = box_at(ytop, 0), tp = box_at(ytop, 1);
@@ -531,6 +532,11 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
     const long XYP = XP * (bs1 + 2 * GP), VP = XYP * (bs2 + 2 * GP), OP = GP + XP * GP + XYP * GP;
     const long XYR = XR * (bs1 + 2 * GR), VR = XYR * (bs2 + 2 * GR), OR = GR + XR * GR + XYR * GR;
     const long XYO = XO * (bs1 + 2 * GO), VO = XYO * (bs2 + 2 * GO), OO = GO + XO * GO + XYO * GO;
+    // this lane's column in each array, from column 0 of the wave's first box (the
+    // wave's boxes are stored one after another)
+    const int lb = lane / BW, lx = lane % BW;
+    const int lp = BW == 64 ? lane : lx + lb * (int)VP, lr = BW == 64 ? lane : lx + lb * (int)VR,
+              lo = BW == 64 ? lane : lx + lb * (int)VO;
     // pointers to the first tile row (row i = 2) of each row class of plane Z:
     // row i of the class is at that pointer + X (i - 2); all uniform
 #define PM_ROW_BASES(X, XY, V, O0, Z, PT, PM, PB)                                              \
@@ -590,7 +596,7 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
             long ot, om, ob;
             PM_ROW_BASES(XP, XYP, VP, OP, Z, ot, om, ob)
 #pragma unroll
-            for (int i = 0; i < NR; i++) { d[i] = pin[(i < 2 ? ot : (i < RY + 2 ? om : ob)) + XP * (i - 2) + lane]; }
+            for (int i = 0; i < NR; i++) { d[i] = pin[(i < 2 ? ot : (i < RY + 2 ? om : ob)) + XP * (i - 2) + lp]; }
             if constexpr (IN == 2) {
                 // plus the constant prolongation of the coarse correction, rounded as
                 // k_prolong_const_box rounds it: the cells fineInterp would leave
@@ -626,7 +632,7 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
 #pragma unroll
         for (int j = 0; j < NQ; j++) {
             const int i = j + 1;
-            d[j] = rhs[(i < 2 ? ot : (i < RY + 2 ? om : ob)) + XR * (i - 2) + lane];
+            d[j] = rhs[(i < 2 ? ot : (i < RY + 2 ? om : ob)) + XR * (i - 2) + lr];
         }
     };
     const bool edge = lane == 0 || lane == 63;
@@ -673,7 +679,7 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
                 (void)ob;
 #pragma unroll
                 for (int r = 0; r < RY; r++) {
-                    const long o = om + XO * r + (side ? 64 : -1);
+                    const long o = om + XO * r + lo + (side ? 1 : -1);
                     const TO v = side ? ef[k & 1][wr][0][r] : ef[k & 1][wl][1][r];
                     if constexpr (OUT == 1) {
                         pacc[o] = v;
@@ -722,7 +728,7 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
             (void)ob;
 #pragma unroll
             for (int r = 0; r < RY; r++) {
-                const long o = om + XO * r + lane;
+                const long o = om + XO * r + lo;
                 if constexpr (OUT == 1) {
                     pacc[o] = pacc[o] + (double)P[S0][r + 2];
                 } else {
@@ -732,6 +738,12 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
                         pout[o] = P[S0][r + 2];
                     }
                     if (GO == 1 && edge) { ef[k & 1][w][side][r] = P[S0][r + 2]; }
+                    if constexpr (GO == 1 && NB > 1) {
+                        // x ghost cells where two of the wave's boxes meet
+                        const T below = lane_shift<kShr1>(P[S0][r + 2], P[S0][r + 2]);
+                        const T above = lane_shift<kShl1>(P[S0][r + 2], P[S0][r + 2]);
+                        if (!edge && (lx == 0 || lx == BW - 1)) { pout[lx == 0 ? o - 1 : o + 1] = lx == 0 ? below : above; }
+                    }
                 }
             }
         }
@@ -2198,6 +2210,8 @@ int pm_layout_create(pm_layout** out, int dim, const int domain[3], const int bo
         set_error("pm_layout_create: upload failed");
         return PM_ERR_HIP;
     }
+    L->x_pairs = L->nb[0] % 2 == 0;
+    for (size_t i = 0; i + 1 < table.size() && L->x_pairs; i += 2) { L->x_pairs = table[i] >= 0 && table[i + 1] == table[i] + 1; }
     *out = L;
     return PM_OK;
 }
@@ -2344,10 +2358,21 @@ namespace pm {
 // sweep, 2 / 3 / 4 the row-register sweep with 4 / 8 / 2 rows per thread.
 static int g_sweep_form = 0;
 
+// boxes 32 cells wide whose x neighbours 2 i, 2 i + 1 follow each other in storage:
+// the row sweep with 4 rows per thread holds two of them in a wave, one lane offset
+// per array.  The tile sweep of such a level stages every plane through LDS with a
+// halo of 4 columns in 36: FP64 solve of 256^3 in 32^3 boxes 10.57 ms with it,
+// 8.33 ms with the rows (both with the block passes below 80^3)
+static bool rows_pairs(const pm_layout* L)
+{
+    return L->bs[0] == 32 && L->nb[0] % 2 == 0 && L->nb[0] <= 16 && L->x_pairs && L->bs[1] % 4 == 0 && L->bs[2] >= 2;
+}
+
 // the row-register sweep takes boxes 64 cells wide, at most 8 across the
-// domain, whose height the rows per thread divide
+// domain, whose height the rows per thread divide, and rows_pairs
 static bool rows_ok(const pm_layout* L, int ry)
 {
+    if (ry == 4 && rows_pairs(L)) { return true; }
     return L->bs[0] == 64 && L->nb[0] <= 8 && L->bs[1] % ry == 0 && L->bs[1] >= 2 && L->bs[2] >= 2;
 }
 
@@ -2360,7 +2385,8 @@ static int g_rows_zc_max = 0, g_rows_nt = -1;
 static int rows_zc(const pm_layout* L, int ry, long waves = kRowsWaves)
 {
     int zc = L->bs[2];
-    while (zc % 2 == 0 && zc > kZcFloor && (long)(L->domain[1] / ry) * (L->domain[2] / zc) * L->nb[0] < waves) { zc /= 2; }
+    const long nw = L->domain[0] / 64;
+    while (zc % 2 == 0 && zc > kZcFloor && (long)(L->domain[1] / ry) * (L->domain[2] / zc) * nw < waves) { zc /= 2; }
     while (g_rows_zc_max > 0 && zc > g_rows_zc_max && zc % 2 == 0) { zc /= 2; }
     return zc;
 }
@@ -2384,12 +2410,12 @@ static int rows_ghosts(const int in_ghost[3], const int out_ghost[3], const int 
     return -1;
 }
 
-template<typename T, int RY, int PF>
+template<typename T, int RY, int PF, int BW>
 static void launch_rows(const pm_layout* L, int in_mode, int ghosts, const T* pi, T* po, const T* rhs,
                         const Lap<T>& c, T lt, double* acc, const pm_layout* C, const T* crs, hipStream_t stream)
 {
     const int zc = rows_zc(L, RY);
-    const dim3 grid((unsigned)((L->domain[1] / RY) * (L->domain[2] / zc))), block((unsigned)(64 * L->nb[0]));
+    const dim3 grid((unsigned)((L->domain[1] / RY) * (L->domain[2] / zc))), block((unsigned)L->domain[0]);
     const LayoutDev D = ldev(L), DC = in_mode == 2 ? ldev(C) : D;
     // non-temporal write-out where the output has no ghost layer (512^3 FP32
     // sweep 0.385 vs 0.392 ms, FP64 0.672 vs 0.691 ms); into ghost-1 arrays
@@ -2397,7 +2423,7 @@ static void launch_rows(const pm_layout* L, int in_mode, int ghosts, const T* pi
     // later complete the same lines in L2
     const bool nt = g_rows_nt < 0 ? true : g_rows_nt == 1;
 #define PM_ROWS(I, O, N, GP, GO)                                                                                  \
-    hipLaunchKernelGGL((k_gsrb_rows<T, RY, I, O, N, GP, 0, GO, PF>), grid, block, 0, stream, D, pi, po, rhs, c, lt, zc, \
+    hipLaunchKernelGGL((k_gsrb_rows<T, RY, I, O, N, GP, 0, GO, PF, BW>), grid, block, 0, stream, D, pi, po, rhs, c, lt, zc, \
                        acc, DC, crs)
 #define PM_ROWS_NT(I, O, GP, GO) \
     if (nt) {                    \
@@ -2445,7 +2471,7 @@ static void sweep_rows(const pm_layout* L, int ry, int ghosts, const void* phi_i
         // FP32 into the scratch level: two cells per lane where the level is an
         // even number of boxes wide (z chunks start on even planes)
         const int zc = rows_zc(L, 4);
-        if (g_sweep_form == 0 && ry == 4 && ghosts == 10 && !acc && L->nb[0] % 2 == 0 && zc % 2 == 0) {
+        if (g_sweep_form == 0 && ry == 4 && ghosts == 10 && !acc && L->bs[0] == 64 && L->nb[0] % 2 == 0 && zc % 2 == 0) {
             const dim3 grid((unsigned)((L->domain[1] / 4) * (L->domain[2] / zc))), block((unsigned)(32 * L->nb[0]));
             const LayoutDev D = ldev(L), DC = in_mode == 2 ? ldev(C) : D;
             const bool nt = g_rows_nt < 0 ? true : g_rows_nt == 1;
@@ -2467,12 +2493,14 @@ static void sweep_rows(const pm_layout* L, int ry, int ghosts, const void* phi_i
     // PF 1: planes loaded one step ahead (two steps ahead measured no faster:
     // 512^3 FP32 sweep 0.387 vs 0.390 ms, back into ghost 1 0.401 vs 0.393 ms,
     // FP64 0.692 vs 0.680 ms)
-    if (ry == 4) {
-        launch_rows<T, 4, 1>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
+    if (L->bs[0] == 32) {
+        launch_rows<T, 4, 1, 32>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
+    } else if (ry == 4) {
+        launch_rows<T, 4, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
     } else if (ry == 2) {
-        launch_rows<T, 2, 1>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
+        launch_rows<T, 2, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
     } else {
-        launch_rows<T, 8, 1>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
+        launch_rows<T, 8, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
     }
 }
 
@@ -2496,7 +2524,7 @@ int level_sweep_restrict(const pm_layout* L, const pm_layout* C, int dtype, cons
         return PM_ERR_UNSUPPORTED;
     };
     if (g_sweep_form != 0) { return unsupported("a sweep form is forced"); }
-    if (L->dim != 3 || rows_ghosts(in_ghost, out_ghost, rhs_ghost, 0) != 1 || !rows_ok(L, 4) || L->bs[1] < 4 ||
+    if (L->dim != 3 || rows_ghosts(in_ghost, out_ghost, rhs_ghost, 0) != 1 || L->bs[0] != 64 || !rows_ok(L, 4) || L->bs[1] < 4 ||
         L->bs[2] < 4 || !box_aligned(L, C)) {
         return unsupported("level shape");
     }
@@ -2587,6 +2615,8 @@ int level_gsrb_sweep_in(const pm_layout* L, int dtype, const void* phi_in, const
             // the prolongation input reads a coarse level with one ghost layer (checked box-aligned above)
             const G3 gcc = g3(coarse_ghost);
             for (int k = 0; k < 3; k++) { coarse_ok = coarse_ok && gcc.g[k] == 1; }
+            // a wave's 64 columns lie over one coarse box
+            coarse_ok = coarse_ok && (L->bs[0] == 64 || C->bs[0] % 32 == 0);
         }
         if (g_sweep_form != 1 && coarse_ok && ghosts > 0 && (!acc || ghosts == 1) && rows_ok(L, ry)) {
             if (dtype == PM_F64) {
