@@ -266,17 +266,21 @@ int pm_level_gsrb(const pm_layout* layout, int dtype, void* phi, const int phi_g
  * of other boxes are read from their owners.  Bitwise the exchange / red /
  * exchange / black sequence.  3-D, periodic layouts covering their domain;
  * PM_ERR_UNSUPPORTED otherwise (use pm_level_gsrb).  Levels of boxes 64 cells
- * wide (at most 8 across the domain) run the row-register kernel, others the
- * LDS tile kernel; both give the same bits. */
+ * wide (at most 8 across the domain; it also writes the x ghost cells of a
+ * ghost-1 phi_out) or 32 (at most 16, an even number, neighbours along x one
+ * after the other in the layout) run the row-register kernel, others the LDS
+ * tile kernel; both give the same bits. */
 int pm_level_gsrb_sweep(const pm_layout* L, int dtype, const void* phi_in, const int in_ghost[3], void* phi_out,
                         const int out_ghost[3], const void* rhs, const int rhs_ghost[3], double dx,
                         pm_stream_t stream);
 /* Which kernel runs the one-pass sweep here and in the multigrid driver
  * (process-wide; tests and benchmarks compare them): 0 automatic (levels of
- * 64-wide boxes: the row-register kernel; FP32 into a ghost-free output two
+ * 64-wide and paired 32-wide boxes: the row-register kernel; FP32 into a ghost-free output two
  * cells per lane where the level is an even number of boxes across, FP32 back
  * into a ghost-1 phi with 8 rows per thread; in the multigrid driver the FP32
- * second pre-smoothing sweep also writes the residual restriction), 1 the LDS
+ * second pre-smoothing sweep also writes the residual restriction, levels that
+ * live in cache take both sweeps and the transfer in one pass, and the last
+ * levels run in one launch), 1 the LDS
  * tile kernel, 2 / 3 / 4 the row-register kernel with 4 / 8 / 2 rows per
  * thread (one cell per lane, restriction in its own pass).
  * pm_level_sweep_tune: the row kernel's largest planes per workgroup (0
@@ -394,7 +398,8 @@ typedef struct pm_mg_options {
     int fused;      /* GSRB sweeps as one out-of-place pass each (pm_level_gsrb_sweep, same
                        bits; 3-D periodic levels) instead of exchange / red / exchange / black;
                        one-box levels of up to 4096 cells run all sweeps of a relaxation in
-                       one launch (same bits) */
+                       one launch, and levels that live in cache both sweeps and the
+                       transfer in one pass (same bits) */
     int inner;      /* precision 1: FP32 V-cycles per refinement step (the preconditioner; 0 or
                        1 = one, at most 4); each starts from the previous one's correction */
 } pm_mg_options;
@@ -428,8 +433,8 @@ int pm_mg_resnorm(pm_mg* mg, void* phi, const void* rhs, double* out_host, pm_st
  * valid extents sizes[3b..3b+2] (box-local indices from 0) and `ghost` ghost
  * layers; ghosted storage holds the boxes one after another (x fastest over
  * [-ghost, n+ghost)), valid storage likewise over [0, n).  Each operator is
- * ONE launch over all boxes (a table of tiles, or a work queue that resets
- * itself) instead of Proto's launch per box (e.g. LevelMultigridSolverImplem.H:
+ * ONE launch over all boxes (a table of tiles, or for the LDS-tile sweep a
+ * work queue that resets itself) instead of Proto's launch per box (e.g. LevelMultigridSolverImplem.H:
  * 366-378), so it can be graph-captured. */
 typedef struct pm_batch pm_batch;
 int pm_batch_create(pm_batch** out, int nboxes, const int* sizes_host, int ghost);
@@ -440,9 +445,9 @@ int pm_batch_offsets(const pm_batch* batch, size_t* ghosted_off, size_t* valid_o
 /* Tiling knobs of the batched operators (what pm_batch_autotune searches):
  * z planes per apply tile (0 = whole box; until pm_batch_configure sets it,
  * chosen from the batch's size), workgroups per CU for the apply (accepted and
- * kept, but without effect: the apply runs one workgroup per tile), rows per GSRB tile (fewer when an FP64 tile as wide as the widest
- * box would not fit the 64 KiB LDS of a workgroup), workgroups per CU for
- * the sweep. */
+ * kept, but without effect: the apply runs one workgroup per tile), rows per
+ * GSRB tile (fewer when an FP64 tile as wide as the widest box would not fit
+ * the 64 KiB LDS of a workgroup), workgroups per CU for the sweep. */
 typedef struct pm_batch_config {
     int apply_zplanes, apply_blocks_per_cu, gsrb_rows, gsrb_blocks_per_cu;
 } pm_batch_config;

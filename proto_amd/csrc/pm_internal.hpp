@@ -34,12 +34,14 @@ int layout_lows(const pm_layout* L, int* lows);
 // box-aligned), the cells pm_level_prolong_add(interp 0) would have left in
 // phi_in, which is not written.  acc (FP32 sweeps, in_mode 0): phi_out is not
 // written; the result is added to the FP64 array acc (layout and ghosts of
-// phi_out) as pm_level_add_correction adds it.  PM_ERR_UNSUPPORTED where the
-// one-pass sweep does not apply.
+// phi_out) as pm_level_add_correction adds it.  x_ghosts: the row sweep of
+// 32-wide boxes may write the x ghost cells of phi_out (their periodic images),
+// which completes its rows' lines; the C entry leaves them as they are.
+// PM_ERR_UNSUPPORTED where the one-pass sweep does not apply.
 int level_gsrb_sweep_in(const pm_layout* L, int dtype, const void* phi_in, const int in_ghost[3], void* phi_out,
                         const int out_ghost[3], const void* rhs, const int rhs_ghost[3], double dx, int in_mode,
                         const pm_layout* C, const void* coarse, const int coarse_ghost[3], hipStream_t stream,
-                        double* acc = nullptr);
+                        double* acc = nullptr, bool x_ghosts = true);
 // nsweeps GSRB sweeps (pm_level_gsrb's colouring and arithmetic, bit for bit)
 // of a one-box periodic 3-D level of at most 4096 cells in one launch, in
 // place; in_mode as level_gsrb_sweep_in (1 zero guess, 2 + constant

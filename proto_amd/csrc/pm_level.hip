@@ -492,7 +492,7 @@ template<typename T, int RY, int IN, int OUT, int NT, int GP, int GR, int GO, in
 __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restrict__ pin, T* __restrict__ pout,
                                                    const T* __restrict__ rhs, Lap<T> c, T lambda, int zc,
                                                    double* __restrict__ pacc, LayoutDev C,
-                                                   const T* __restrict__ crs)
+                                                   const T* __restrict__ crs, int xg)
 {
     constexpr int NR = RY + 4;  // phi rows held: Y0 - 2 .. Y0 + RY + 1
     constexpr int NQ = RY + 2;  // rhs rows: Y0 - 1 .. Y0 + RY
@@ -672,7 +672,7 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
     // against 0.728 ms at 512^3
     auto ghost_cols = [&](int k) {
         if constexpr (GO == 1 && OUT == 0) {
-            if (edge) {
+            if (edge && (BW == 64 || xg)) {
                 long ot, om, ob;
                 PM_ROW_BASES(XO, XYO, VO, OO, k, ot, om, ob)
                 (void)ot;
@@ -742,7 +742,7 @@ __global__ __launch_bounds__(512) void k_gsrb_rows(LayoutDev L, const T* __restr
                         // x ghost cells where two of the wave's boxes meet
                         const T below = lane_shift<kShr1>(P[S0][r + 2], P[S0][r + 2]);
                         const T above = lane_shift<kShl1>(P[S0][r + 2], P[S0][r + 2]);
-                        if (!edge && (lx == 0 || lx == BW - 1)) { pout[lx == 0 ? o - 1 : o + 1] = lx == 0 ? below : above; }
+                        if (xg && !edge && (lx == 0 || lx == BW - 1)) { pout[lx == 0 ? o - 1 : o + 1] = lx == 0 ? below : above; }
                     }
                 }
             }
@@ -2412,7 +2412,8 @@ static int rows_ghosts(const int in_ghost[3], const int out_ghost[3], const int 
 
 template<typename T, int RY, int PF, int BW>
 static void launch_rows(const pm_layout* L, int in_mode, int ghosts, const T* pi, T* po, const T* rhs,
-                        const Lap<T>& c, T lt, double* acc, const pm_layout* C, const T* crs, hipStream_t stream)
+                        const Lap<T>& c, T lt, double* acc, const pm_layout* C, const T* crs, bool xg,
+                        hipStream_t stream)
 {
     const int zc = rows_zc(L, RY);
     const dim3 grid((unsigned)((L->domain[1] / RY) * (L->domain[2] / zc))), block((unsigned)L->domain[0]);
@@ -2424,7 +2425,7 @@ static void launch_rows(const pm_layout* L, int in_mode, int ghosts, const T* pi
     const bool nt = g_rows_nt < 0 ? true : g_rows_nt == 1;
 #define PM_ROWS(I, O, N, GP, GO)                                                                                  \
     hipLaunchKernelGGL((k_gsrb_rows<T, RY, I, O, N, GP, 0, GO, PF, BW>), grid, block, 0, stream, D, pi, po, rhs, c, lt, zc, \
-                       acc, DC, crs)
+                       acc, DC, crs, xg ? 1 : 0)
 #define PM_ROWS_NT(I, O, GP, GO) \
     if (nt) {                    \
         PM_ROWS(I, O, 1, GP, GO); \
@@ -2456,7 +2457,7 @@ static void launch_rows(const pm_layout* L, int in_mode, int ghosts, const T* pi
 template<typename T>
 static void sweep_rows(const pm_layout* L, int ry, int ghosts, const void* phi_in, void* phi_out,
                        const void* rhs, double dx, int in_mode, const pm_layout* C, const void* coarse,
-                       hipStream_t stream, double* acc)
+                       hipStream_t stream, double* acc, bool xg)
 {
     double lam = -(dx * dx) / (4.0 * L->dim);
     lam *= 2.0;
@@ -2494,13 +2495,13 @@ static void sweep_rows(const pm_layout* L, int ry, int ghosts, const void* phi_i
     // 512^3 FP32 sweep 0.387 vs 0.390 ms, back into ghost 1 0.401 vs 0.393 ms,
     // FP64 0.692 vs 0.680 ms)
     if (L->bs[0] == 32) {
-        launch_rows<T, 4, 1, 32>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
+        launch_rows<T, 4, 1, 32>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, xg, stream);
     } else if (ry == 4) {
-        launch_rows<T, 4, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
+        launch_rows<T, 4, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, xg, stream);
     } else if (ry == 2) {
-        launch_rows<T, 2, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
+        launch_rows<T, 2, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, xg, stream);
     } else {
-        launch_rows<T, 8, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, stream);
+        launch_rows<T, 8, 1, 64>(L, in_mode, ghosts, pi, (T*)phi_out, (const T*)rhs, c, lt, acc, C, (const T*)coarse, xg, stream);
     }
 }
 
@@ -2569,7 +2570,7 @@ int level_sweep_restrict(const pm_layout* L, const pm_layout* C, int dtype, cons
 int level_gsrb_sweep_in(const pm_layout* L, int dtype, const void* phi_in, const int in_ghost[3], void* phi_out,
                         const int out_ghost[3], const void* rhs, const int rhs_ghost[3], double dx, int in_mode,
                         const pm_layout* C, const void* coarse, const int coarse_ghost[3], hipStream_t stream,
-                        double* acc)
+                        double* acc, bool x_ghosts)
 {
     PM_REQUIRE(L && phi_out && rhs && (phi_in || in_mode == 1), "pm_level_gsrb_sweep: bad argument");
     PM_REQUIRE(!acc || (dtype == PM_F32 && in_mode == 0), "pm_level_gsrb_sweep: the FP64 accumulation is for FP32 sweeps");
@@ -2620,9 +2621,9 @@ int level_gsrb_sweep_in(const pm_layout* L, int dtype, const void* phi_in, const
         }
         if (g_sweep_form != 1 && coarse_ok && ghosts > 0 && (!acc || ghosts == 1) && rows_ok(L, ry)) {
             if (dtype == PM_F64) {
-                sweep_rows<double>(L, ry, ghosts, phi_in, phi_out, rhs, dx, in_mode, C, coarse, stream, acc);
+                sweep_rows<double>(L, ry, ghosts, phi_in, phi_out, rhs, dx, in_mode, C, coarse, stream, acc, x_ghosts);
             } else {
-                sweep_rows<float>(L, ry, ghosts, phi_in, phi_out, rhs, dx, in_mode, C, coarse, stream, acc);
+                sweep_rows<float>(L, ry, ghosts, phi_in, phi_out, rhs, dx, in_mode, C, coarse, stream, acc, x_ghosts);
             }
             PM_CHECK_LAUNCH();
             return PM_OK;
@@ -2752,7 +2753,7 @@ int pm_level_gsrb_sweep(const pm_layout* L, int dtype, const void* phi_in, const
 {
     PM_REQUIRE(phi_in, "pm_level_gsrb_sweep: bad argument");
     return level_gsrb_sweep_in(L, dtype, phi_in, in_ghost, phi_out, out_ghost, rhs, rhs_ghost, dx, 0, nullptr, nullptr,
-                               nullptr, S(stream), nullptr);
+                               nullptr, S(stream), nullptr, false);
 }
 
 int pm_level_jacobi(const pm_layout* L, int dtype, void* phi, const int phi_ghost[3], const void* rhs,

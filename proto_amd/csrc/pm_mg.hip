@@ -140,7 +140,8 @@ static int relax(pm_mg* mg, int l, int dtype, void* phi, const void* rhs, void* 
                 }
             }
             if (rc != PM_OK) {
-                rc = pm_level_gsrb_sweep(L.layout, dtype, phi, mg->g1, tmp, mg->g0, rhs, mg->g0, L.dx, s);
+                rc = level_gsrb_sweep_in(L.layout, dtype, phi, mg->g1, tmp, mg->g0, rhs, mg->g0, L.dx, 0, nullptr,
+                                         nullptr, nullptr, s);
                 if (rc == PM_ERR_UNSUPPORTED) { break; }
                 if (rc != PM_OK) { return rc; }
             }
@@ -155,7 +156,8 @@ static int relax(pm_mg* mg, int l, int dtype, void* phi, const void* rhs, void* 
                                            nullptr, nullptr, s, acc64));
                 *folded = true;
             } else if (!(restricted && *restricted)) {
-                MG_TRY(pm_level_gsrb_sweep(L.layout, dtype, tmp, mg->g0, phi, mg->g1, rhs, mg->g0, L.dx, s));
+                MG_TRY(level_gsrb_sweep_in(L.layout, dtype, tmp, mg->g0, phi, mg->g1, rhs, mg->g0, L.dx, 0, nullptr,
+                                           nullptr, nullptr, s));
             }
         }
     }

@@ -258,9 +258,9 @@ def test_row_sweep_equals_tile_sweep(dt, domain, box):
 @pytest.mark.parametrize("domain,box", [((64, 32, 32), (32, 32, 32)), ((512, 8, 12), (32, 4, 6)),
                                         ((192, 64, 96), (32, 32, 32)), ((128, 40, 16), (32, 20, 16))])
 def test_row_sweep_of_paired_boxes(dt, domain, box):
-    """Boxes 32 cells wide, two to a wave: the tile sweep's bits, x ghost cells
-    of the outputs included, for one to eight waves across; a layout in another
-    order, whose x neighbours do not follow each other, gives the same cells."""
+    """Boxes 32 cells wide, two to a wave: the tile sweep's bits, ghost cells
+    left as they were, for one to eight waves across; a layout in another
+    order, whose x neighbours do not follow each other, gives the same."""
     t = np.float64 if dt == pa.PM_F64 else np.float32
     h, lows = _box_layout(domain, box)
     nbox = len(lows)
@@ -280,17 +280,14 @@ def test_row_sweep_of_paired_boxes(dt, domain, box):
             for k in range(2):
                 pa.call("pm_level_gsrb_sweep", lay, dt, vp(a), G1, vp(tmp), G0, vp(rh), G0, 1.0 / domain[0], None)
                 pa.call("pm_level_gsrb_sweep", lay, dt, vp(tmp), G0, vp(a), G1, vp(rh), G0, 1.0 / domain[0], None)
-            if key != "rows":
-                pa.call("pm_level_exchange", lay, dt, vp(a), G1, 1, None)
             inv = np.argsort(perm) if key == "perm" else slice(None)
             outs[key] = (host(a).reshape(nbox, box[2] + 2, box[1] + 2, box[0] + 2)[inv], host(tmp).reshape(nbox, e0)[inv])
     finally:
         pa.call("pm_level_sweep_form", 0)
         pa.lib().pm_layout_destroy(h)
         pa.lib().pm_layout_destroy(hp)
-    rows = (slice(None), slice(1, -1), slice(1, -1))
     for key in ("rows", "perm"):
-        assert outs[key][0][rows].tobytes() == outs["tile"][0][rows].tobytes(), key
+        assert outs[key][0].tobytes() == outs["tile"][0].tobytes(), key
         assert outs[key][1].tobytes() == outs["tile"][1].tobytes(), key
 
 
