@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "pm_block.hpp"
+#include "pm_fas_grid.hpp"
 #include "pm_layout.hpp"
 
 struct pm_fas {
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(256) void k_fas_relax(LayoutDev L, G3 gu, G3 gf, co
 // Rows per wave: 2 measured fastest at 512^3 in 64^3 boxes (FAS solve 0.450 s,
 // against 0.463 s with 1 row and 0.475 / 0.496 s with 4 / 3 rows): 4 rows held
 // the relaxation at 3 waves per SIMD by both registers and LDS.
-constexpr int FZ_RY = 2, FZ_TY = 4 * FZ_RY, FZ_NE = (FZ_TY + 4) * 68;
+constexpr int FZ_NE = (FZ_TY + 4) * 68;
 
 // IN = 2 (with NB): the staged input is u + the constant prolongation of the
 // coarse correction crs (layout C, ghost gc), rounded as fineCorrect's
@@ -928,8 +929,6 @@ __global__ __launch_bounds__(256) void k_fas_delta(LayoutDev C, G3 gc, G3 g0, co
     }
 }
 
-static unsigned fas_blocks(long n) { return (unsigned)std::min<long>((n + 255) / 256, 1024); }
-
 #define FAS_TRY(x)                    \
     do {                              \
         int rc_ = (x);                \
@@ -938,9 +937,7 @@ static unsigned fas_blocks(long n) { return (unsigned)std::min<long>((n + 255) /
 
 static const int G2[3] = {2, 2, 2}, G0[3] = {0, 0, 0};
 
-// boxes the z-marching operator kernel takes: 32..64 cells wide, at least a tile
-// tall and deep
-static bool fz_ok(const LayoutDev& D) { return D.bs[0] >= 32 && D.bs[0] <= 64 && D.bs[1] >= 16 && D.bs[2] >= 8; }
+static bool fz_ok(const LayoutDev& D) { return fz_box(D.bs); }
 // levels whose z-marching operator can read the neighbouring boxes instead of
 // the ghost layer: periodic, every box present, fewer than 2^31 elements
 static bool fz_nb(const pm_layout* L)
@@ -953,18 +950,11 @@ static bool fz_nb(const pm_layout* L)
     return gvol(D, g3(G2)) * L->nboxes < (1L << 31);
 }
 
-// its grid: 8-row tiles (16 rows of 32-wide boxes) x z chunks (halved while fewer than
-// 2048 workgroups) x boxes
 static dim3 fz_grid(const LayoutDev& D, int* zc)
 {
-    const int ty = D.bs[0] <= 32 ? 2 * FZ_TY : FZ_TY, nyt = (D.bs[1] + ty - 1) / ty;
-    auto blocks = [&](int z) { return (long)nyt * ((D.bs[2] + z - 1) / z) * D.nboxes; };
-    int z = D.bs[2];
-    while (z > 8 && blocks(z) < 2048) { z = (z + 1) / 2; }
-    // 128^3 cells: 4 planes 9.1 ms a solve, 8 planes 9.8; 192^3: 13.4 against 12.6
-    if (z > 4 && z <= 8 && blocks(z) < 1024) { z = (z + 1) / 2; }
-    *zc = z;
-    return dim3((unsigned)(nyt * ((D.bs[2] + z - 1) / z)), (unsigned)D.nboxes);
+    const FzGrid g = fz_grid(D.bs, D.nboxes);
+    *zc = g.zc;
+    return dim3(g.blocks, (unsigned)D.nboxes);
 }
 
 // n Jacobi relaxations of level l.  delta (the coarse correction of level
@@ -1163,12 +1153,12 @@ static int fas_resnorm(pm_fas* M, void* u, const void* f, double* out, hipStream
     const LayoutDev D = ldev(Lv.layout);
     const bool nb = in_solve && fz_nb(Lv.layout);
     if (!nb) { FAS_TRY(pm_level_exchange(Lv.layout, PM_F64, u, G2, 1, s)); }
-    const long cells = (long)D.bs[0] * D.bs[1] * D.bs[2];
-    unsigned bpb = fas_blocks(cells);
+    const unsigned bpb = fas_norm_blocks(D.bs, D.nboxes);
+    PM_REQUIRE((size_t)bpb * D.nboxes <= M->cap_part, "pm_fas: %u partials a box and %d boxes, room for %zu", bpb, D.nboxes,
+               M->cap_part);
     if (fz_ok(D)) {
         int zc = 0;
         const dim3 zgrid = fz_grid(D, &zc);
-        bpb = zgrid.x;  // no more partials than the generic kernel's (<= 64 per box)
         if (nb) {
             hipLaunchKernelGGL((k_fas_op_z<1, 1>), zgrid, dim3(256), 0, s, D, (const double*)u, (const double*)f,
                                (double*)nullptr, fas_coefs(Lv.dx), M->d_part, res_out, zc, D, g3(G0),
@@ -1269,7 +1259,6 @@ int pm_fas_create(pm_fas** out, const pm_layout* fine, int num_levels, double dx
         rc = pm_layout_create(&M->lv[l].layout, 3, dom, box, fine->periodic, (int)(lows.size() / 3), lows.data());
         M->lv[l].dx = M->lv[l - 1].dx * 2;
     }
-    size_t maxpart = 0;
     for (int l = 0; l < num_levels && rc == PM_OK; l++) {
         auto& L = M->lv[l];
         const LayoutDev D = ldev(L.layout);
@@ -1278,9 +1267,10 @@ int pm_fas_create(pm_fas** out, const pm_layout* fine, int num_levels, double dx
         if (l > 0 && rc == PM_OK) { rc = fas_alloc(M, &L.phi, 8 * e2); }
         if (l > 0 && rc == PM_OK) { rc = fas_alloc(M, &L.f, 8 * e0); }
         if (l > 0 && rc == PM_OK) { rc = fas_alloc(M, &L.phi0, 8 * e0); }
-        if (l == 0) { maxpart = (size_t)fas_blocks((long)e0 / D.nboxes) * D.nboxes; }
     }
-    if (rc == PM_OK) { rc = fas_alloc(M, (void**)&M->d_part, 8 * std::max<size_t>(maxpart, 1)); }
+    // the norm is taken on the finest level: one partial per workgroup of its kernel
+    M->cap_part = (size_t)fas_norm_blocks(fine->bs, fine->nboxes) * fine->nboxes;
+    if (rc == PM_OK) { rc = fas_alloc(M, (void**)&M->d_part, 8 * M->cap_part); }
     if (rc == PM_OK && hipHostMalloc((void**)&M->h_norm, 64, hipHostMallocDefault) != hipSuccess) {
         set_error("pm_fas_create: pinned host allocation failed");
         M->h_norm = nullptr;

@@ -118,6 +118,35 @@ def test_fas_resnorm_equals_residual_norm():
     pa.call("pm_fas_destroy", fas)
 
 
+@pytest.mark.parametrize("bs", [(64, 320, 128), (48, 384, 96), (32, 512, 192), (64, 256, 256), (40, 24, 20)])
+def test_fas_norm_of_unequal_boxes(bs):
+    """One box of unequal extents, whose norm kernel launches more workgroups than a
+    per-cell kernel would (and one whose does not): the norm is the maximum over
+    every one of them, wherever it lies, and the solve runs."""
+    lay, fas = ctypes.c_void_p(), ctypes.c_void_p()
+    pa.call("pm_layout_create", ctypes.byref(lay), 3, pa.i3(bs), pa.i3(bs), pa.i3([1] * 3), 1, pa.i3([0] * 3))
+    pa.call("pm_fas_create", ctypes.byref(fas), lay, 2, 1.0 / bs[0])
+    n = int(np.prod(bs))
+    say("fas norm", bs)
+    phi = zeros(int(np.prod([b + 4 for b in bs])))
+    f = util.uniform(94, 1, n)
+    r1, r2 = ctypes.c_double(), ctypes.c_double()
+    for at in (0, n // 2, n - 1):
+        g = f.copy()
+        g[at] = -7.0  # phi is zero, so the residual is the force
+        f_d, res = dev(g), zeros(n)
+        pa.call("pm_fas_residual", fas, vp(phi), vp(f_d), vp(res), ctypes.byref(r2), None)
+        pa.call("pm_fas_resnorm", fas, vp(phi), vp(f_d), ctypes.byref(r1), None)
+        assert r1.value == r2.value == 7.0 and host(res).tobytes() == g.tobytes()
+    g = f - f.mean()
+    f_d, hist, it = dev(g), np.zeros(3), ctypes.c_int()
+    pa.call("pm_fas_solve", fas, vp(phi), vp(f_d), 2, 0.0, hist.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
+            ctypes.byref(it), None)
+    assert it.value == 2 and hist[0] == np.abs(g).max() and np.all(np.isfinite(hist)) and hist[2] < hist[0]
+    pa.call("pm_fas_destroy", fas)
+    pa.call("pm_layout_destroy", lay)
+
+
 def test_tune_table_round_trip():
     coefs, offs, *_ = util.lib_stencil("Laplacian", 0, 3, np.float64)
     st = pa.Stencil(coefs, offs, pa.PM_F64)
