@@ -29,10 +29,8 @@ inline FzGrid fz_grid(const int bs[3], long nboxes)
     auto blocks = [&](int z) { return (long)nyt * ((bs[2] + z - 1) / z) * nboxes; };
     int z = bs[2];
     while (z > 8 && blocks(z) < 2048) { z = (z + 1) / 2; }
-    // 128^3 cells: 4 planes 9.1 ms a solve, 8 planes 9.8; 192^3: 13.4 against 12.6.
-    // Chunks of 6 and 5 stay: 3 would be odd, and only even chunks hold whole coarse
-    // cells, which the fused coarse force needs.
-    if ((z == 7 || z == 8) && blocks(z) < 1024) { z = 4; }
+    // 128^3 cells: 4 planes 9.1 ms a solve, 8 planes 9.8; 192^3: 13.4 against 12.6
+    if (z > 4 && z <= 8 && blocks(z) < 1024) { z = (z + 1) / 2; }
     return FzGrid{z, (unsigned)(nyt * ((bs[2] + z - 1) / z))};
 }
 

@@ -59,16 +59,3 @@ def test_norm_partials_cover_the_launch(grids):
         most = max(most, launched / cellwise)
     assert most > 1  # boxes whose launch outgrows the per-cell count are among them
     assert grids([(64, 320, 128, 1), (64, 256, 512, 1)]) == [(1, 4, 1280, 1280, 1024), (1, 8, 2048, 2048, 1024)]
-
-
-def test_chunks_hold_whole_coarse_cells(grids):
-    """The shortest chunks are even wherever the halvings of the box depth are: an odd
-    one takes the coarse force off the z-marching kernel."""
-    todo = [(x, y, z, n) for x in (32, 48, 64) for y in (16, 32, 48, 64) for z in (8, 12, 16, 24, 28, 32, 48, 56, 64, 96, 192)
-            for n in (1, 2, 4, 8, 27, 64)]
-    for (x, y, z, n), (fz, zc, blocks, held, cellwise) in zip(todo, grids(todo)):
-        halved = z
-        while halved > 8 and halved > zc:
-            halved = (halved + 1) // 2
-        assert zc % 2 == 0 or halved % 2 == 1, (x, y, z, n, zc)
-    assert [g[1] for g in grids([(48, 48, 48, 1), (48, 48, 48, 8), (64, 64, 64, 1), (48, 96, 56, 1)])] == [6, 6, 4, 4]
