@@ -1067,6 +1067,16 @@ static bool fas_block_ok(const pm_fas* M, int l)
     // 32^3 boxes, 128^3 cells (17 cycles) 12261 / 12254 / 13983, 48^3 boxes, 96^3
     // cells 5687 / 5983 / -, but 16^3 boxes (whose other form is an exchange and a
     // per-cell kernel a sweep), 128^3 cells 16842 / 16818 / 14625
+    // A tile costs about the same (0.2 us of the chip) whatever its size, one sweep a
+    // launch a time per stored cell, so levels that split into many small or ragged tiles
+    // keep the latter.  us of a cycle, one sweep a launch -> two: 20^3 boxes 80^3 cells
+    // 444 -> 423, 120^3 681 -> 877; 26^3 boxes 104^3 cells 474 -> 550; 12^3 boxes 96^3
+    // cells 681 -> 534; 6^3 boxes 96^3 cells 1004 -> 909, 120^3 1255 -> 1502; 4^3 boxes
+    // 32^3 cells 263 -> 230, 48^3 413 -> 435, 128^3 2298 -> 5358.
+    int nt[3], t[3];
+    block_tiles(L->bs, L->nboxes, nt, t);
+    const long tiles = (long)nt[0] * nt[1] * nt[2] * L->nboxes;
+    if (tiles > 500 + gvol(ldev(L), g3(G2)) * L->nboxes / 1136) { return false; }
     const long side = fz_ok(ldev(L)) ? 72 : 160;
     return cells <= side * side * side;
 }

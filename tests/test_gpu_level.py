@@ -612,6 +612,20 @@ def test_fas_block_levels_vs_oracle(n, bs, levels):
     assert phi.tobytes() == ophi.tobytes()
 
 
+@pytest.mark.parametrize("n,bs,levels", [(32, 4, 2), (48, 4, 2)])
+def test_fas_small_boxes_vs_oracle(n, bs, levels):
+    """Boxes of 4^3 cells on both sides of the count of tiles from which the
+    relaxations go one a launch again: two a launch (512 tiles), one (1728)."""
+    say("fas small boxes", n, bs, levels)
+    force = util.gaussian_rhs(n, 5, 17)
+    it, hist, phi = _fas(n, bs, levels, force, maxiter=3)
+    ophi, ohist = np.zeros(n ** 3), np.zeros(5)
+    oit = util.oracle().orc_fas_solve(n, levels, util.ptr(force), util.ptr(ophi), 3, 1e-10, util.ptr(ohist))
+    assert it == oit
+    assert hist.tobytes() == ohist[:oit + 1].tobytes()
+    assert phi.tobytes() == ophi.tobytes()
+
+
 @pytest.mark.parametrize("dt", [pa.PM_F64, pa.PM_F32])
 @pytest.mark.parametrize("bs,ghost,ncomp", [(4, (1, 1, 1), 1), (4, (4, 4, 4), 5), (6, (2, 0, 3), 4), (8, (0, 3, 1), 3),
                                             (10, (3, 1, 2), 8), (4, (5, 5, 5), 2)])
