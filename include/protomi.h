@@ -630,9 +630,11 @@ int pm_server_restore(pm_server* srv, const void* buffer_host, size_t bytes, pm_
  * by the stream.  A capture records that buffer's address, so a buffer seen
  * by a capture is never freed when a later, larger call grows the scratch:
  * it is kept until pm_stream_destroy, and graphs captured on a stream must
- * not be launched after that stream is destroyed.  A call that would need
- * more scratch than the stream holds while it is capturing fails with
- * PM_ERR_UNSUPPORTED (run it once on the stream before capturing). */
+ * not be launched after that stream is destroyed.  A captured call that
+ * needs more than the buffer takes a 1 MiB reserve, which comes with the
+ * stream's first scratch; one that needs more than that, or captures on a
+ * stream that has no scratch yet, fails with PM_ERR_UNSUPPORTED (run it once
+ * on the stream before capturing). */
 typedef void* pm_graph_t;
 int pm_graph_begin(pm_stream_t stream);
 int pm_graph_end(pm_stream_t stream, pm_graph_t* graph);

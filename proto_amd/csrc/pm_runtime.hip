@@ -26,13 +26,18 @@ void set_error(const char* fmt, ...)
 // caller's own capture).  Such a buffer is never freed on growth: it moves to
 // the stream's retired list and is released only by pm_stream_destroy.
 // Buffers never seen by a capture are freed on growth after the stream
-// drains, as before.
+// drains, as before.  A capture can grow nothing, so a reserve that holds the
+// partials of any automatically tiled stencil reduction of up to 32768
+// workgroups comes with a stream's first scratch and serves the captured calls
+// that the buffer is too small for.  It stays until pm_stream_destroy.
 struct WsEntry {
     void* ptr = nullptr;
+    void* reserve = nullptr;
     size_t bytes = 0;
     bool captured = false;       // handed out while the stream was capturing
     std::vector<void*> retired;  // superseded buffers a graph may still use
 };
+constexpr size_t kWsReserve = (size_t)1 << 20;
 static std::mutex g_ws_mu;
 static std::map<hipStream_t, WsEntry>* g_ws = nullptr;
 
@@ -54,9 +59,14 @@ int workspace(hipStream_t stream, size_t bytes, void** out)
     const bool capturing = stream_capturing(stream);
     if (bytes > w.bytes) {
         if (capturing) {
+            if (w.reserve && bytes <= kWsReserve) {
+                *out = w.reserve;
+                return PM_OK;
+            }
             // neither a stream drain nor an allocation may be recorded into a graph
             set_error("workspace: %zu bytes of per-stream scratch needed under graph capture, %zu available; "
-                      "run the call once on the stream before capturing it", bytes, w.bytes);
+                      "run the call once on the stream before capturing it", bytes,
+                      w.reserve ? std::max(w.bytes, kWsReserve) : w.bytes);
             return PM_ERR_UNSUPPORTED;
         }
         if (w.ptr) {
@@ -70,9 +80,11 @@ int workspace(hipStream_t stream, size_t bytes, void** out)
             w.bytes = 0;
             w.captured = false;
         }
-        // at least 96 KiB: the partials of a fused residual of up to about 200^3
-        // cells (3072 workgroups), so that a stream warmed by any call captures it
-        size_t nb = bytes < ((size_t)96 << 10) ? ((size_t)96 << 10) : bytes;
+        if (!w.reserve && hipMalloc(&w.reserve, kWsReserve) != hipSuccess) {
+            (void)hipGetLastError();  // without it a capture finds only the buffer
+            w.reserve = nullptr;
+        }
+        size_t nb = bytes < ((size_t)1 << 16) ? ((size_t)1 << 16) : bytes;
         hipError_t e = hipMalloc(&w.ptr, nb);
         if (e != hipSuccess) {
             set_error("workspace hipMalloc(%zu): %s", nb, hipGetErrorString(e));
@@ -110,6 +122,7 @@ static void workspace_release(hipStream_t stream)
     if (it == g_ws->end()) { return; }
     (void)hipStreamSynchronize(stream);
     if (it->second.ptr) { (void)hipFree(it->second.ptr); }
+    if (it->second.reserve) { (void)hipFree(it->second.reserve); }
     for (void* p : it->second.retired) { (void)hipFree(p); }
     g_ws->erase(it);
 }

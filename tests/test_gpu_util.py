@@ -326,3 +326,56 @@ def test_scratch_growth_under_capture_is_refused():
     pa.call("pm_graph_destroy", g)
     assert rc == -4
     assert b"under graph capture" in pa.lib().pm_last_error()
+
+
+@pytest.mark.parametrize("what,n", [("residual2", (5, 16384, 9)), ("residual", (3, 8192, 100)),
+                                    ("apply_reduce", (2, 16384, 200))])
+def test_thin_boxes_capture_on_a_stream_with_small_scratch(what, n):
+    """Thin boxes, whose automatic tiles are many for their cells, capture on a
+    stream whose only scratch comes from a small call; every replay gives the
+    eager call's bits, with eager calls between the replays."""
+    from proto_amd.device import Stream
+    s = Stream()
+    st = {k: pa.Stencil(*util.lib_stencil(k)[:2]) for k in ("Laplacian", "Laplacian_19", "Laplacian_27")}
+    cells = n[0] * n[1] * n[2]
+    ub, rb = pa.Box.of([-1] * 3, list(n)), pa.Box.of([0] * 3, [v - 1 for v in n])
+    u = dev(util.uniform(81, 0, (n[0] + 2) * (n[1] + 2) * (n[2] + 2)))
+    f, r1, r2, red = dev(util.uniform(81, 1, cells)), zeros(cells), zeros(cells), zeros(4)
+    small, out = dev(util.uniform(81, 2, 1000)), zeros(1)
+
+    def call():
+        if what == "residual2":
+            return pa.lib().pm_stencil_residual2(st["Laplacian"].h, st["Laplacian_27"].h, vp(u), ctypes.byref(ub),
+                                                 vp(f), vp(r1), vp(r2), ctypes.byref(rb), 1.0, 1.0, vp(red), s.h)
+        if what == "residual":
+            return pa.lib().pm_stencil_residual(st["Laplacian"].h, vp(u), ctypes.byref(ub), vp(f), vp(r1),
+                                                ctypes.byref(rb), 1.0, vp(red), s.h)
+        return pa.lib().pm_stencil_apply_reduce(st["Laplacian_19"].h, vp(u), ctypes.byref(ub), vp(r1), ctypes.byref(rb),
+                                                ctypes.byref(rb), 1, 1.0, pa.RED_SUM, vp(red), 0, s.h)
+
+    def warm():
+        pa.call("pm_reduce", pa.RED_ABS, pa.PM_F64, vp(small), 1000, vp(out), 0, s.h)
+    pa.call("pm_stream_sync", None)
+    warm()
+    s.sync()
+    say("thin capture", what, n)
+    g = ctypes.c_void_p()
+    pa.call("pm_graph_begin", s.h)
+    rc = call()
+    pa.call("pm_graph_end", s.h, ctypes.byref(g))
+    assert rc == 0, pa.lib().pm_last_error()
+    got = []
+    for _ in range(3):
+        for a in (r1, r2, red):
+            pa.call("pm_memset_zero", vp(a), a.nbytes, s.h)
+        pa.call("pm_graph_launch", g, s.h)
+        warm()  # the stream's own scratch, between the replays
+        s.sync()
+        got.append([host(a).tobytes() for a in (r1, r2, red)])
+    pa.call("pm_graph_destroy", g)
+    for a in (r1, r2, red):
+        pa.call("pm_memset_zero", vp(a), a.nbytes, s.h)
+    assert call() == 0
+    s.sync()
+    want = [host(a).tobytes() for a in (r1, r2, red)]
+    assert got == [want] * 3
