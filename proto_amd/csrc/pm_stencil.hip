@@ -71,9 +71,10 @@ static int detect_kind(const pm_stencil* s)
 // flight.  Points z + 1 .. z + R - 1 and the neighbouring rows find most taps
 // in L1; the workgroups of an XCD walk z first, so the planes shared between
 // groups of R are re-read from its L2.  Bound by memory: CellToFace of order 4
-// on 128^3 x 5 FP64,
-// 168 MB a direction: 36 us (4.7 TB/s) against 62 with one point a thread, its
-// position from 64-bit divisions and the tap list read from memory.
+// on 128^3 x 5 FP64, 168 MB a direction: 36 us (4.7 TB/s) against 62 with one
+// point a thread, its position from 64-bit divisions and the tap list read from
+// memory.  FLAT (R = 1): the position runs over the whole component, planes
+// included, so boxes of few cells a plane fill their waves too.
 constexpr int kDirectTaps = 32;  // taps held in the arguments; longer lists are read from the handle
 
 template<typename T>
@@ -81,8 +82,9 @@ struct DirectArgs {
     const T* src;
     T* dst;
     long nx, ncell;              // index points per row / per plane
+    long n;                      // positions of a component: ncell (FLAT: all its points)
     int nz, nzg, ntap, replace;
-    unsigned nch;                // 256-point chunks per plane
+    unsigned nch, b0;            // 256-position chunks per plane (FLAT: component); first workgroup of this launch
     long sx, sy, sz, dx, dy, dz; // elements per index step
     long scomp, dcomp;           // elements per component
     T c[kDirectTaps];            // coefficients, pre-scaled
@@ -93,24 +95,30 @@ struct DirectArgs {
     T scale;
 };
 
-template<typename T, int R, bool WIDE, bool LISTS>
+template<typename T, int R, bool FLAT, bool WIDE, bool LISTS>
 __global__ __launch_bounds__(256) void k_direct(DirectArgs<T> a)
 {
+    static_assert(!FLAT || R == 1, "a flat position holds one point");
     using O = std::conditional_t<WIDE, size_t, unsigned>;
-    unsigned b = xcd_remap(blockIdx.x, gridDim.x);
-    const int z0 = (int)(b % a.nzg) * R;
-    b /= a.nzg;
-    const O cell = (O)(b % a.nch) * 256 + threadIdx.x;
+    unsigned b = a.b0 + xcd_remap(blockIdx.x, gridDim.x);
+    int z0 = 0;
+    if constexpr (!FLAT) {
+        z0 = (int)(b % a.nzg) * R;
+        b /= a.nzg;
+    }
+    const O pos = (O)(b % a.nch) * 256 + threadIdx.x;
     const int comp = (int)(b / a.nch);
-    if (cell >= (O)a.ncell) { return; }
+    if (pos >= (O)a.n) { return; }
+    const O zf = FLAT ? pos / (O)a.ncell : 0, cell = pos - zf * (O)a.ncell;
     const O y = cell / (O)a.nx, x = cell - y * (O)a.nx;
-    const O so = (x * (O)a.sx + y * (O)a.sy) * (O)sizeof(T), dof = (x * (O)a.dx + y * (O)a.dy) * (O)sizeof(T);
+    const O so = (x * (O)a.sx + y * (O)a.sy + zf * (O)a.sz) * (O)sizeof(T),
+            dof = (x * (O)a.dx + y * (O)a.dy + zf * (O)a.dz) * (O)sizeof(T);
     const T* s[R];
     T* d[R];
     T acc[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const long z = min(z0 + r, a.nz - 1);
+        const long z = FLAT ? 0 : min(z0 + r, a.nz - 1);
         s[r] = a.src + (comp * a.scomp + z * a.sz);
         d[r] = reinterpret_cast<T*>(reinterpret_cast<char*>(a.dst + (comp * a.dcomp + z * a.dz)) + dof);
         acc[r] = a.replace ? (T)0 : *d[r];
@@ -720,22 +728,42 @@ static int launch_direct(const pm_stencil* st, const void* src, const Box3& sbox
             a.off[j] = st->offs[3 * j] + st->offs[3 * j + 1] * sx + st->offs[3 * j + 2] * sxy;
         }
     }
-    // in-plane byte offsets within 32 bits (a plane of less than 4 GB) but for huge planes
-    const long span = std::max((a.nx - 1) * a.sx + (box_ny(ibox) - 1) * a.sy, (a.nx - 1) * a.dx + (box_ny(ibox) - 1) * a.dy);
-    const bool wide = (span + 1) * (long)sizeof(T) >= (1L << 32) || a.ncell + 256 >= (1L << 32);
-    // four planes a thread; one where there are fewer (2-D)
-    const int R = a.nz >= 4 && !wide ? 4 : 1;
-    a.nzg = (a.nz + R - 1) / R;
-    const long nch = (a.ncell + 255) / 256, blocks = nch * a.nzg * ncomp;
-    a.nch = (unsigned)nch;
-    PM_REQUIRE(blocks < (1L << 31), "pm_stencil_apply: index box too large for one launch");
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, a); };
-    if (wide) {
-        if (lists) { go(k_direct<T, 1, true, true>); } else { go(k_direct<T, 1, true, false>); }
-    } else if (R == 1) {
-        if (lists) { go(k_direct<T, 1, false, true>); } else { go(k_direct<T, 1, false, false>); }
-    } else {
-        if (lists) { go(k_direct<T, 4, false, true>); } else { go(k_direct<T, 4, false, false>); }
+    const long ny = box_ny(ibox), elem = (long)sizeof(T), nzg = (a.nz + 3) / 4;
+    auto nch = [](long n) { return (n + 255) / 256; };
+    // Four planes a thread, but one point at a flat position where there are fewer
+    // planes, where a plane would leave most of its waves' lanes idle, where rows are so
+    // short that neighbouring lanes share no lines, and where the launch would be short
+    // of waves.  us, four planes / flat: 48 taps FP32, 24^3 10.7 / 8.5, 96^3 23.3 / 42.7,
+    // 4 x 4 x 65536 96 / 39, 8 x 8 x 16384 28.6 / 48.6; FP64 1 x 300 x 300 20.0 / 10.9,
+    // 2000 x 2000 x 1 357 / 178; four taps along x FP64 4 x 4 x 65536 17.5 / 7.9, 128^3 x 5
+    // 36 / 46.
+    const long waves = (a.ncell + 63) / 64 * nzg * ncomp;
+    bool flat = a.nz < 4 || a.nx < 3 || a.ncell < 32 || waves < 768;
+    // byte offsets of the position within 32 bits (a component, FLAT, or a plane of less than 4 GB)
+    auto fits = [&](long z) {
+        const long span = std::max((a.nx - 1) * a.sx + (ny - 1) * a.sy + z * a.sz,
+                                   (a.nx - 1) * a.dx + (ny - 1) * a.dy + z * a.dz);
+        return (span + 1) * elem < (1L << 32) && a.ncell * (z + 1) + 256 < (1L << 32);
+    };
+    flat = flat || !fits(0);
+    const bool wide = flat && !fits(a.nz - 1);
+    a.n = flat ? a.ncell * a.nz : a.ncell;
+    a.nzg = flat ? 1 : (int)nzg;
+    a.nch = (unsigned)nch(a.n);
+    const long blocks = nch(a.n) * a.nzg * ncomp, most = 1L << 23;
+    PM_REQUIRE(blocks < (1L << 32), "pm_stencil_apply: index box too large");
+    // a launch holds fewer than 2^32 threads
+    for (long b0 = 0; b0 < blocks; b0 += most) {
+        a.b0 = (unsigned)b0;
+        const unsigned nb = (unsigned)std::min(most, blocks - b0);
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, s, a); };
+        if (!flat) {
+            if (lists) { go(k_direct<T, 4, false, false, true>); } else { go(k_direct<T, 4, false, false, false>); }
+        } else if (wide) {
+            if (lists) { go(k_direct<T, 1, true, true, true>); } else { go(k_direct<T, 1, true, true, false>); }
+        } else {
+            if (lists) { go(k_direct<T, 1, true, false, true>); } else { go(k_direct<T, 1, true, false, false>); }
+        }
     }
     PM_CHECK_LAUNCH();
     return PM_OK;

@@ -11,6 +11,7 @@ import pytest
 import proto_amd as pa
 import util
 from gpu_util import box, config2_inputs, dev, empty, host, say, vp, zeros
+from proto_amd.device import DeviceArray
 from test_oracle import merge
 
 pytestmark = pytest.mark.gpu
@@ -154,6 +155,79 @@ def test_wide_and_ratio_stencils_vs_oracle(dtype, ntap):
             ref[q * nd:(q + 1) * nd] = r
         out = apply_gpu(st, src, slo, shi, dst0.copy(), dlo, dhi, lo, hi, replace, scale, ncomp=2)
         assert out.tobytes() == ref.tobytes(), trial
+
+
+@pytest.mark.parametrize("dtype", [pa.PM_F64, pa.PM_F32])
+@pytest.mark.parametrize("n", [(66, 70, 41), (64, 3, 300), (3, 90, 130), (2, 90, 130), (31, 1, 900), (32, 1, 900),
+                               (300, 301, 4), (300, 301, 3)])
+def test_generic_kernel_forms_vs_oracle(dtype, n):
+    """Both forms of the generic kernel (four planes a thread, flat positions) on
+    both sides of the lines between them, in arguments and in lists, two
+    components; bitwise."""
+    npdt = np.float64 if dtype == pa.PM_F64 else np.float32
+    rng = np.random.default_rng(5 + n[0])
+    pool = np.array([(x, y, z) for z in range(-2, 3) for y in range(-2, 3) for x in range(-2, 3)], dtype=np.int32)
+    lo, hi = np.array([0, 0, 0]), np.array(n) - 1
+    slo, shi, dlo, dhi = lo - 2, hi + 3, lo - 1, hi + 1
+    ns, nd = util.box_size(slo, shi), util.box_size(dlo, dhi)
+    src, dst0 = util.uniform(910, 0, 2 * ns).astype(npdt), util.uniform(910, 1, 2 * nd).astype(npdt)
+    for ntap, replace in ((5, True), (37, False)):
+        o = pool[rng.permutation(len(pool))[:ntap]].copy()
+        o[0] = (2, -2, 1)
+        c = rng.uniform(-2, 2, size=ntap).astype(npdt)
+        st = pa.Stencil(c, o, dtype, 3)
+        say("forms", dtype, n, ntap)
+        ref = dst0.copy()
+        for q in range(2):
+            r = ref[q * nd:(q + 1) * nd].copy()
+            util.oracle_apply(c, o, src[q * ns:(q + 1) * ns].copy(), slo, shi, r, dlo, dhi, lo, hi, replace, 1.0)
+            ref[q * nd:(q + 1) * nd] = r
+        out = apply_gpu(st, src, slo, shi, dst0.copy(), dlo, dhi, lo, hi, replace, 1.0, ncomp=2)
+        assert out.tobytes() == ref.tobytes(), ntap
+
+
+def _apply_in_parts_cancels(st, src, sb, dst, n, parts):
+    """dst = st(src) in one call, then minus the same in parts: +0 everywhere if both
+    give the same bits (one tap, so a product and its negative)."""
+    db = pa.Box.of([0] * 3, [v - 1 for v in n])
+    cells = n[0] * n[1] * n[2]
+    out = zeros(1, np.float32)
+    pa.call("pm_fill_uniform", pa.PM_F32, vp(dst), cells, 1, 0, 0.0, 7.0, None)
+    pa.call("pm_stencil_apply", st.h, vp(src), ctypes.byref(sb), vp(dst), ctypes.byref(db), ctypes.byref(db), 1, 1, 1.0, None)
+    pa.call("pm_reduce", pa.RED_MIN, pa.PM_F32, vp(dst), cells, vp(out), 0, None)
+    assert -2.5 <= host(out)[0] < -2.4  # the values, which fill (-2.5, 2.5)
+    for lo, hi in parts:
+        ib = pa.Box.of(lo, hi)
+        pa.call("pm_stencil_apply", st.h, vp(src), ctypes.byref(sb), vp(dst), ctypes.byref(db), ctypes.byref(ib), 1, 0, -1.0,
+                None)
+    pa.call("pm_reduce", pa.RED_ABS, pa.PM_F32, vp(dst), cells, vp(out), 0, None)
+    assert host(out)[0] == 0.0
+
+
+def test_index_box_of_more_positions_than_a_launch_holds():
+    """A 2-D index box of more than 2^32 points, in one call and in quarters."""
+    n = (65540, 65540, 1)
+    st = pa.Stencil(np.array([2.5], dtype=np.float32), np.array([[3, 0, 0]], dtype=np.int32), pa.PM_F32)
+    pa.call("pm_stencil_set_kind", st.h, 0)
+    sb = pa.Box.of([0, 0, 0], [n[0] + 2, n[1] - 1, 0])
+    src, dst = DeviceArray((n[0] + 3) * n[1], np.float32), DeviceArray(n[0] * n[1], np.float32)
+    pa.call("pm_fill_uniform", pa.PM_F32, vp(src), src.n, 23, 0, 1.0, 0.0, None)
+    say("large 2-D box", n)
+    ys = [0, 16385, 32770, 49155, 65540]
+    _apply_in_parts_cancels(st, src, sb, dst, n, [([0, a, 0], [n[0] - 1, b - 1, 0]) for a, b in zip(ys, ys[1:])])
+
+
+def test_index_box_of_a_component_beyond_4_gb():
+    """A thin and tall index box whose positions lie more than 4 GB apart, in one
+    call and in parts that do not."""
+    n, st = (4, 4, 18000), pa.Stencil(np.array([2.5], dtype=np.float32), np.array([[0, 3, 0]], dtype=np.int32), pa.PM_F32,
+                                      3, (1, 1, 64))
+    sb = pa.Box.of([0, 0, 0], [31, 31, 64 * n[2] - 1])
+    src, dst = DeviceArray(32 * 32 * 64 * n[2], np.float32), DeviceArray(n[0] * n[1] * n[2], np.float32)
+    pa.call("pm_fill_uniform", pa.PM_F32, vp(src), src.n, 24, 0, 1.0, 0.0, None)
+    say("tall box", n)
+    zs = [0, 6000, 12000, 18000]
+    _apply_in_parts_cancels(st, src, sb, dst, n, [([0, 0, a], [3, 3, b - 1]) for a, b in zip(zs, zs[1:])])
 
 
 @pytest.mark.parametrize("name", ["Laplacian", "Laplacian_27"])
