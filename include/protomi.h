@@ -443,9 +443,10 @@ int pm_batch_elems(const pm_batch* batch, size_t* ghosted, size_t* valid);
 /* nboxes + 1 element offsets of every box in ghosted / valid storage. */
 int pm_batch_offsets(const pm_batch* batch, size_t* ghosted_off, size_t* valid_off);
 /* Tiling knobs of the batched operators (what pm_batch_autotune searches):
- * z planes per apply tile (0 = whole box; until pm_batch_configure sets it,
- * chosen from the batch's size), workgroups per CU for the apply (accepted and
- * kept, but without effect: the apply runs one workgroup per tile), rows per
+ * z planes per apply tile (0, which a new batch has = chosen from the batch's
+ * size; as many as the tallest box or more = whole boxes), workgroups per CU for
+ * the apply (accepted and kept, but without effect: the apply runs one workgroup
+ * per tile), rows per
  * GSRB tile (fewer when an FP64 tile as wide as the widest box would not fit
  * the 64 KiB LDS of a workgroup), workgroups per CU for the sweep. */
 typedef struct pm_batch_config {

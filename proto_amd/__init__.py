@@ -303,6 +303,7 @@ class Batch:
         self.voff = list(vo)
 
     def configure(self, apply_zplanes=0, gsrb_rows=8, blocks_per_cu=4, gsrb_blocks_per_cu=None):
+        """apply_zplanes 0: chosen from the batch's size."""
         c = BatchConfig(apply_zplanes, blocks_per_cu, gsrb_rows,
                         blocks_per_cu if gsrb_blocks_per_cu is None else gsrb_blocks_per_cu)
         call("pm_batch_configure", self.h, ctypes.byref(c))

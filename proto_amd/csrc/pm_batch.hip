@@ -40,7 +40,7 @@ struct pm_batch {
     std::vector<size_t> goff, voff;  // nboxes + 1
     void* d_boxes = nullptr;         // BatchBox[nboxes]
     void* d_items = nullptr;         // BatchItem[] (apply), one workgroup each
-    int nitems_apply = 0, apply_tz = -1;  // apply_tz -1: the z chunk of apply_auto_zc
+    int nitems_apply = 0, apply_tz = -1;  // apply_tz: the cfg.apply_zplanes the items are built for
     void* d_gitems = nullptr;        // BatchItem[] (gsrb)
     int nitems_gsrb = 0, gsrb_rows = 0;
     unsigned* d_counter = nullptr;   // queue head, blocks done (LDS-ring sweep)
@@ -1098,19 +1098,20 @@ int apply_auto_zc(const pm_batch* B)
     return (int)std::min(24L, std::max(4L, planes / 1024));
 }
 
-// Apply items: the tiles of every box in z chunks of tz (0 = whole box, -1 =
-// apply_auto_zc).  Each XCD's list takes its boxes largest first.
+// Apply items: the tiles of every box in z chunks of tz (0 = apply_auto_zc).  Each
+// XCD's list takes its boxes largest first.
 int build_apply_items(pm_batch* B, int tz)
 {
-    const int zauto = tz < 0 ? apply_auto_zc(B) : tz;
+    const int zc = tz > 0 ? tz : apply_auto_zc(B);
     const auto xb = boxes_by_xcd(B);
     std::vector<std::vector<BatchItem>> lists(kXcd);
     for (int x = 0; x < kXcd; x++) {
         for (int b : xb[x]) {
-            const int nz = B->sizes[3 * b + 2], zc = zauto > 0 ? zauto : nz;
-            for (int z0 = 0; z0 < nz; z0 += zc) {
+            const int nz = B->sizes[3 * b + 2];
+            for (int z0 = 0, z1; z0 < nz; z0 = z1) {
+                z1 = z0 + std::min(zc, nz - z0);
                 apply_tiles(B, b, [&](int x0, int xw, int y0, int tr) {
-                    lists[x].push_back(BatchItem{b, x0, y0, z0, std::min(nz, z0 + zc), tr, xw, 0});
+                    lists[x].push_back(BatchItem{b, x0, y0, z0, z1, tr, xw, 0});
                 });
             }
         }
@@ -1267,7 +1268,7 @@ int pm_batch_create(pm_batch** out, int nboxes, const int* sizes_host, int ghost
     int rc = upload(&B->d_boxes, boxes.data(), sizeof(BatchBox) * nboxes);
     if (rc == PM_OK && hipMalloc((void**)&B->d_counter, 2 * sizeof(unsigned)) != hipSuccess) { rc = PM_ERR_NOMEM; }
     if (rc == PM_OK && hipMemset(B->d_counter, 0, 2 * sizeof(unsigned)) != hipSuccess) { rc = PM_ERR_HIP; }
-    if (rc == PM_OK) { rc = build_apply_items(B, -1); }
+    if (rc == PM_OK) { rc = build_apply_items(B, B->cfg.apply_zplanes); }
     if (rc == PM_OK) { rc = build_gsrb_items(B, B->cfg.gsrb_rows); }
     B->rows_ok = true;
     B->pairs_ok = ghost % 2 == 0;
@@ -1601,7 +1602,9 @@ int pm_batch_autotune(pm_batch* B, const pm_stencil* st, const void* src, void* 
         *ms /= (float)reps;
         return PM_OK;
     };
-    const int zs[] = {0, 8, 16, 32, apply_auto_zc(B)};
+    int tallest = 0;
+    for (int b = 0; b < B->nboxes; b++) { tallest = std::max(tallest, B->sizes[3 * b + 2]); }
+    const int zs[] = {0, 8, 16, 32, tallest};
     const int bpcs[] = {1, 2, 4, 8};
     const int rows[] = {2, 4, 8, 16};
     pm_batch_config win = keep;

@@ -354,3 +354,65 @@ def test_batch_short_z_chunks_vs_oracle(dt, widths):
     B.gsrb(dt, vp(s_d), vp(p_d), vp(r_d), 1.0 / 32)
     got, want = host(p_d), oracle_gsrb_batch(B, src, rhs, 1.0 / 32)
     assert first_diff(B, got, want, False) is None, first_diff(B, got, want, False)
+
+
+class _KernelNode(ctypes.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                ("grid", ctypes.c_uint * 3), ("params", ctypes.c_void_p), ("lds", ctypes.c_uint)]
+
+
+def launched(stream, call):
+    """Workgroups (x) of every kernel that call(stream) launches, from a capture that is not run."""
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the library's own runtime, already loaded
+    graph, n = ctypes.c_void_p(), ctypes.c_size_t()
+    assert hip.hipStreamBeginCapture(stream.h, 0) == 0
+    try:
+        call()
+    finally:
+        assert hip.hipStreamEndCapture(stream.h, ctypes.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+    grids = []
+    for node in nodes:
+        p = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        grids.append(p.grid[0])
+    assert hip.hipGraphDestroy(graph) == 0
+    return grids
+
+
+def test_batch_configuration_round_trip():
+    """Writing back the configuration that was read, changing another field of it, and
+    an autotuning that fails leave the apply its automatic tiles."""
+    from proto_amd.device import Stream
+    B = make_batch([(16 + 8 * (i % 3), 24, 20 + 4 * (i % 5)) for i in range(20)])
+    c, o, *_ = util.lib_stencil("Laplacian_27", 0, 3, np.float64)
+    st = pa.Stencil(c, o, pa.PM_F64)
+    s, src, dst = Stream(), zeros(B.ghosted_elems), zeros(B.valid_elems)
+
+    def tiles():
+        return launched(s, lambda: B.apply(st, vp(src), vp(dst), 1.0, s.h))
+    first = tiles()
+    say("batch tiles", first)
+    assert len(first) == 1 and first[0] > 20 * 3  # several z chunks a box
+    cfg = B.config()
+    pa.call("pm_batch_configure", B.h, ctypes.byref(cfg))
+    assert tiles() == first
+    cfg.gsrb_rows = 4
+    pa.call("pm_batch_configure", B.h, ctypes.byref(cfg))
+    assert tiles() == first and B.config().gsrb_rows == 4
+    B.configure(gsrb_rows=16)
+    assert tiles() == first
+    B.configure(apply_zplanes=1 << 30)  # whole boxes
+    whole = tiles()
+    assert whole[0] < first[0]
+    B.configure(apply_zplanes=8)
+    assert whole[0] < tiles()[0]
+    B.configure()
+    assert tiles() == first
+    nineteen = pa.Stencil(*util.lib_stencil("Laplacian_19", 0, 3, np.float64)[:2], pa.PM_F64)
+    out, rhs = zeros(B.ghosted_elems), zeros(B.valid_elems)
+    with pytest.raises(pa.NativeError):  # the apply takes the 7- and 27-point shapes only
+        B.autotune(nineteen, vp(src), vp(dst), vp(out), vp(rhs), 1.0)
+    assert tiles() == first
