@@ -1036,6 +1036,8 @@ int upload(void** dptr, const void* host, size_t bytes)
 // largest first, each to the least loaded, so that the tiles of a box share an
 // L2 that serves the halo rows they re-read.
 constexpr int kXcd = 8;
+// Most items of one launch of the apply (256 threads each).
+constexpr int kLaunchItems = 1 << 23;
 std::vector<std::vector<int>> boxes_by_xcd(const pm_batch* B)
 {
     std::vector<int> order(B->nboxes);
@@ -1350,31 +1352,21 @@ int pm_batch_apply(pm_batch* B, const pm_stencil* st, const void* src, void* dst
     int rc = stencil_info(st, &kind, &dtype, &cv);
     if (rc) { return rc; }
     PM_REQUIRE(kind == 7 || kind == 27, "pm_batch_apply: needs the 7-point or 27-point Laplacian shape");
-    const unsigned nb = (unsigned)B->nitems_apply;
+    // a launch holds fewer than 2^32 threads
+    auto go = [&](auto kern, auto tag) {
+        using T = decltype(tag);
+        BCoefs<T> cc;
+        coefs_of<T>(cv, scale, cc);
+        for (int i = 0; i < B->nitems_apply; i += kLaunchItems) {
+            const unsigned nb = (unsigned)std::min(kLaunchItems, B->nitems_apply - i);
+            hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, S(stream), (const BatchBox*)B->d_boxes,
+                               (const BatchItem*)B->d_items + i, B->ghost, (const T*)src, (T*)dst, cc);
+        }
+    };
     if (dtype == PM_F64) {
-        BCoefs<double> cc;
-        coefs_of<double>(cv, scale, cc);
-        if (kind == 7) {
-            hipLaunchKernelGGL((k_batch_apply<double, 7, 1>), dim3(nb), dim3(256), 0, S(stream),
-                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->ghost, (const double*)src,
-                               (double*)dst, cc);
-        } else {
-            hipLaunchKernelGGL((k_batch_apply<double, 27, 1>), dim3(nb), dim3(256), 0, S(stream),
-                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->ghost, (const double*)src,
-                               (double*)dst, cc);
-        }
+        if (kind == 7) { go(k_batch_apply<double, 7, 1>, 0.0); } else { go(k_batch_apply<double, 27, 1>, 0.0); }
     } else {
-        BCoefs<float> cc;
-        coefs_of<float>(cv, scale, cc);
-        if (kind == 7) {
-            hipLaunchKernelGGL((k_batch_apply<float, 7, 1>), dim3(nb), dim3(256), 0, S(stream),
-                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->ghost, (const float*)src,
-                               (float*)dst, cc);
-        } else {
-            hipLaunchKernelGGL((k_batch_apply<float, 27, 1>), dim3(nb), dim3(256), 0, S(stream),
-                               (const BatchBox*)B->d_boxes, (const BatchItem*)B->d_items, B->ghost, (const float*)src,
-                               (float*)dst, cc);
-        }
+        if (kind == 7) { go(k_batch_apply<float, 7, 1>, 0.0f); } else { go(k_batch_apply<float, 27, 1>, 0.0f); }
     }
     PM_CHECK_LAUNCH();
     return PM_OK;

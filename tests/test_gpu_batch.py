@@ -12,6 +12,7 @@ import pytest
 import proto_amd as pa
 import util
 from gpu_util import dev, host, say, vp, zeros
+from proto_amd.device import DeviceArray
 
 pytestmark = pytest.mark.gpu
 
@@ -416,3 +417,31 @@ def test_batch_configuration_round_trip():
     with pytest.raises(pa.NativeError):  # the apply takes the 7- and 27-point shapes only
         B.autotune(nineteen, vp(src), vp(dst), vp(out), vp(rhs), 1.0)
     assert tiles() == first
+
+
+def test_batch_of_more_tiles_than_a_launch_holds():
+    """2^24 + 3 boxes of one cell, one workgroup each: the first and last boxes' bits
+    (a launch holds fewer than 2^24 workgroups of 256 threads)."""
+    n, t = (1 << 24) + 3, np.float32
+    sizes, h = np.ones(3 * n, dtype=np.int32), ctypes.c_void_p()
+    pa.call("pm_batch_create", ctypes.byref(h), n, sizes.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), 1)
+    c, o, *_ = util.lib_stencil("Laplacian", 0, 3, t)
+    st = pa.Stencil(c, o, pa.PM_F32)
+    src, dst = DeviceArray(27 * n, t), DeviceArray(n, t)
+    pa.call("pm_fill_uniform", pa.PM_F32, vp(src), src.n, 61, 0, 1.0, 0.0, None)
+    pa.call("pm_fill_uniform", pa.PM_F32, vp(dst), dst.n, 61, 0, 0.0, 99.0, None)
+    say("batch of", n)
+    pa.call("pm_batch_apply", h, st.h, vp(src), vp(dst), 0.5, None)
+    got = host(dst)
+    k = 2000
+    for first in (0, n // 2, n - k):
+        s = np.zeros(27 * k, dtype=t)
+        pa.call("pm_memcpy", s.ctypes.data_as(ctypes.c_void_p), ctypes.c_void_p(src.ptr.value + 4 * 27 * first), s.nbytes,
+                1, None)
+        pa.call("pm_stream_sync", None)
+        want = np.zeros(k, dtype=t)
+        for b in range(k):
+            util.oracle_apply(c, o, s[27 * b:27 * b + 27].copy(), [-1] * 3, [1] * 3, want[b:b + 1], [0] * 3, [0] * 3,
+                              [0] * 3, [0] * 3, True, 0.5)
+        assert got[first:first + k].tobytes() == want.tobytes(), first
+    pa.call("pm_batch_destroy", h)
