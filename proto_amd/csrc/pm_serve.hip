@@ -880,17 +880,10 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
     // levels below the finest of at most SMALL_CELLS cells relax in one launch
     // each (k_srv_small), all requests' such levels of one depth together
     auto small = [&](const Active& a, int d) { return d > 0 && (long)a.ns[d] * a.ns[d] * a.ns[d] <= SMALL_CELLS; };
-    // From 64^3 cells in flight on, the forms below.  Fewer keep one launch per
-    // operator and 32-plane tiles, though these are the slower ones there too (a
-    // lone 32^3 request: 0.7 ms against more than 1): test_alone_equals_in_mix
-    // holds that a request arriving 1 ms after a 32^3 one still meets it in flight.
-    long cells0 = 0;
-    for (const Active& a : act) { cells0 += (long)a.ns[0] * a.ns[0] * a.ns[0]; }
-    const bool many = cells0 > 64L * 64 * 64;
     // The bottom of a request's hierarchy from depth d on in one launch: a level
     // below the finest of at most 4096 cells, even sizes down to the coarsest.
     auto bottom = [&](const Active& a, int d) {
-        if (!many || !zero_in || !fold_prolong || d >= (int)a.ns.size() || !small(a, d)) { return false; }
+        if (!zero_in || !fold_prolong || d >= (int)a.ns.size() || !small(a, d)) { return false; }
         bool ok = (int)a.ns.size() - d <= kBotLevels;
         for (size_t l = d; l < a.ns.size(); l++) { ok = ok && a.ns[l] % 2 == 0; }
         return ok;
@@ -900,12 +893,13 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
     // one pass (pm_block.hpp); at most 128^3 cells over all requests, as the
     // driver's FP32 levels.  The sweeps of the other depths cut their boxes into
     // chunks of 32, 16 or 8 planes for about 2048 tiles: their time is the z walk
-    // (1.5 us a plane) until the chip is full.
+    // (1.5 us a plane) until the chip is full.  With the bottoms, a request alone,
+    // 32^3 cells 2.27 -> 0.63 ms, 64^3 4.25 -> 0.87, eight of 32^3 2.6 -> 1.1.
     std::vector<char> blk(maxd + 1, 0);
     std::vector<int> zcs(maxd + 1, SZC);
     for (int d = 0; d <= maxd; d++) {
         long cells = 0, cols = 0;
-        const bool ok = many && pre == 2 && post == 2 && zero_in;
+        const bool ok = pre == 2 && post == 2 && zero_in;
         for (const Active& a : act) {
             if (a.fresh || d >= (int)a.ns.size() || bottom(a, d) || below_bottom(a, d)) { continue; }
             const long m = a.ns[d];
@@ -913,7 +907,7 @@ int build_plan(pm_server* S, std::vector<Active>& act, hipStream_t s)
             cols += ((m + sweep_cols((int)m) - 1) / sweep_cols((int)m)) * ((m + SR - 1) / SR) * m;
         }
         blk[d] = ok && cells <= 128L * 128 * 128;
-        while (many && zcs[d] > 8 && cols / zcs[d] < 2048) { zcs[d] /= 2; }
+        while (zcs[d] > 8 && cols / zcs[d] < 2048) { zcs[d] /= 2; }
     }
     auto block = [&](const Active& a, int d) {
         return blk[d] && d < (int)a.ns.size() - 1 && a.ns[d] >= 6 && a.ns[d] % 2 == 0 && !bottom(a, d) && !below_bottom(a, d);

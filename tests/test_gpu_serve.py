@@ -102,10 +102,26 @@ def test_alone_equals_in_mix():
     assert st[3]["iters"] == sa[0]["iters"]
     assert srv.result(3, 48).tobytes() == alone_a.tobytes()
     assert srv.result(1, 32).tobytes() == alone_b.tobytes()
-    # continuous batching: the second arrival (1 ms) joined while the first was
-    # still in flight, and the last (5 ms) while an earlier one still was
-    assert st[1]["admit_s"] < st[0]["finish_s"]
-    assert any(st[5]["admit_s"] < st[j]["finish_s"] for j in range(5))
+
+
+def test_request_joins_while_another_is_in_flight():
+    """Continuous batching, without a clock: two slots, all requests present.  The
+    first converges in fewer cycles than the second, and every request in flight
+    takes a cycle a turn, so the third takes the first's slot while the second is
+    still iterating; its answer and the second's are the ones they have alone."""
+    loose, tight, late = req(64, 4, 30, tol=1e-2), req(64, 9, 31, tol=1e-10), req(48, 7, 21)
+    srv = pa.Server(mode=0)
+    alone = []
+    for r in (tight, late):
+        st = srv.run([r])
+        alone.append((st[0]["iters"], srv.result(0, r["n"]).tobytes()))
+    srv = pa.Server(mode=0, max_active=2)
+    st = srv.run([loose, tight, late])
+    say("joined", [(s["iters"], s["admit_s"], s["finish_s"]) for s in st])
+    assert all(s["status"] == pa.SERVE_SOLVED for s in st)
+    assert st[0]["iters"] < st[1]["iters"]
+    assert st[0]["finish_s"] <= st[2]["admit_s"] < st[1]["finish_s"]
+    assert [(st[i + 1]["iters"], srv.result(i + 1, r["n"]).tobytes()) for i, r in enumerate((tight, late))] == alone
 
 
 def test_plain_mode_is_driver_fp64_and_modes_agree():
