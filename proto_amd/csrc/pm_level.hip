@@ -2291,10 +2291,14 @@ int pm_level_exchange(const pm_layout* L, int dtype, void* data, const int ghost
         // about 4096 workgroups, whose neighbour tables then serve several cells a
         // thread (64^3 cells a box, 64 boxes, FP32 x 2: 37.8 us against 51.3 with one
         // cell a thread); one cell a thread where more than 192 MB move and the reads
-        // in flight count (192^3 in 32^3 boxes, FP64 x 5: 167 against 175)
+        // in flight count (192^3 in 32^3 boxes, FP64 x 5: 167 against 175), but 8192
+        // workgroups where boxes are small (16^3 boxes, 192^3, FP64 x 3, 2 ghost layers:
+        // 135 against 206), and also where a wide box would leave the second turn of its
+        // workgroups mostly empty (64 x 16 x 16, 256 boxes, FP64 x 3: 34 against 60)
         const bool large = (double)nghost * L->nboxes * ncomp * dtype_size(dtype) * 2 > 192e6;
-        const long most = large ? nghost : std::max(1L, 4096L / L->nboxes);
-        const dim3 gnb((unsigned)std::min((nghost + 255) / 256, most), L->nboxes);
+        const long chunks = (nghost + 255) / 256, few = std::max(1L, (large ? 8192L : 4096L) / L->nboxes);
+        const bool single = large ? nghost > 8000 : L->bs[0] >= 32 && 2 * chunks <= 3 * few;
+        const dim3 gnb((unsigned)(single ? chunks : std::min(chunks, few)), L->nboxes);
         PM_DISPATCH_T(dtype, hipLaunchKernelGGL(k_exchange_nb<T>, gnb, dim3(256), 0, S(stream), D, g, (T*)data, ncomp));
         PM_CHECK_LAUNCH();
         return PM_OK;

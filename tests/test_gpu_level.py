@@ -651,3 +651,29 @@ def test_exchange_components_and_ghosts(dt, bs, ghost, ncomp):
     say("exchange", dt, bs, ghost, ncomp)
     pa.call("pm_level_exchange", L.h, dt, vp(d), pa.i3(ghost), ncomp, None)
     assert host(d).tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("bs,k,g", [((4, 4, 4), (16, 16, 16), 2), ((64, 16, 16), (4, 8, 8), 1), ((64, 16, 16), (4, 8, 8), 2),
+                                    ((16, 16, 16), (12, 12, 12), 2), ((24, 20, 12), (2, 3, 2), 4)])
+def test_exchange_over_workgroup_counts(bs, k, g):
+    """Several turns a workgroup and one cell a thread, small boxes by the thousand and
+    wide ones, unequal extents: every ghost cell is its periodic image."""
+    dom = [b * n for b, n in zip(bs, k)]
+    lows = np.array([(x * bs[0], y * bs[1], z * bs[2]) for z in range(k[2]) for y in range(k[1]) for x in range(k[0])],
+                    dtype=np.int32)
+    h = ctypes.c_void_p()
+    pa.call("pm_layout_create", ctypes.byref(h), 3, pa.i3(dom), pa.i3(bs), pa.i3([1] * 3), len(lows),
+            lows.reshape(-1).ctypes.data_as(ctypes.POINTER(ctypes.c_int)))
+    glob = util.uniform(43, 0, dom[0] * dom[1] * dom[2]).reshape(dom[2], dom[1], dom[0])
+    want = np.empty((len(lows), 3) + tuple(b + 2 * g for b in bs[::-1]))
+    for b, lo in enumerate(lows):
+        z, y, x = [np.arange(lo[d] - g, lo[d] + bs[d] + g) % dom[d] for d in (2, 1, 0)]
+        want[b] = glob[z][:, y][:, :, x]
+    want *= np.arange(1, 4)[None, :, None, None, None]
+    data = np.full_like(want, -7)
+    data[:, :, g:-g, g:-g, g:-g] = want[:, :, g:-g, g:-g, g:-g]
+    d = dev(data.reshape(-1))
+    say("exchange", bs, k, g)
+    pa.call("pm_level_exchange", h, pa.PM_F64, vp(d), pa.i3([g] * 3), 3, None)
+    assert host(d).tobytes() == want.tobytes()
+    pa.call("pm_layout_destroy", h)
