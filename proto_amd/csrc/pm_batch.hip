@@ -1174,15 +1174,20 @@ int build_row_items(pm_batch* B, int ry, int cpl, int wpb)
     };
     // Planes per item: the whole box where that already gives about 1536 waves
     // (six a CU; 3072 with one cell per lane, whose waves are shorter), else
-    // shorter chunks, which sweep three planes more than they write.  FP64 pairs
-    // (us, whole boxes -> chunks): 20 boxes 72 -> 10, 100 81 -> 31, 300 130 -> 116,
-    // from 600 boxes on whole; FP32 quads 42 -> 8, 43 -> 16, 47 -> 41.
-    long planes = 0;
+    // shorter chunks, which sweep three planes more than they write; the whole box
+    // too where chunks for that many waves would be within those three planes of
+    // the mean box.  FP64 pairs (us, whole boxes -> chunks): 20 boxes 72 -> 10, 100
+    // 97 -> 39, 300 131 -> 116, 400 149 -> 144, 600 196 -> 211 (not cut); FP32 quads 42
+    // -> 8, 48 -> 20, 62 -> 58, 72 -> 71, 98 -> 107 (not cut).
+    long planes = 0, waves = 0;
     for (int b = 0; b < B->nboxes; b++) {
-        const long nstrips = (B->sizes[3 * b + 1] + ry - 1) / ry, P = per_item(b);
-        planes += wpb * ((nstrips + P - 1) / P) * B->sizes[3 * b + 2];
+        const long nstrips = (B->sizes[3 * b + 1] + ry - 1) / ry, P = per_item(b), w = wpb * ((nstrips + P - 1) / P);
+        waves += w;
+        planes += w * B->sizes[3 * b + 2];
     }
-    const int zc = (int)std::min(4096L, std::max(4L, planes / (cpl == 1 ? 3072 : 1536))) & ~1;
+    const long most = cpl == 1 ? 3072 : 1536;
+    const bool whole = (double)planes / most + 3 >= (double)planes / waves;
+    const int zc = whole ? 4096 : (int)std::min(4096L, std::max(4L, planes / most)) & ~1;
     std::vector<std::vector<RowItem>> lists(kXcd);
     for (int x = 0; x < kXcd; x++) {
         std::stable_sort(xb[x].begin(), xb[x].end(),
