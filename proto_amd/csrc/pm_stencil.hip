@@ -809,14 +809,34 @@ static int auto_tz(const Box3& ibox, int ry)
 //   27-point FP64   10.0 ->  5.5   20.0 -> 20.2  450 -> 388
 //   27-point FP32   13.1 ->  6.0   16.1 -> 14.0  244 -> 217
 //   2 residuals F64 19.2 -> 11.4   36.8 -> 36.2  878 -> 764
-static ZCfg default_cfg(int mode, int dtype, const Box3& ibox)
+// The generic z-march (kind 1) reads its taps from LDS and is bound by that and by
+// the walk, not by halo rows: 4 rows a thread as soon as they leave two workgroups
+// a CU, and 4 planes, 8 on large boxes.  19-point apply (the shape before the rule
+// above / that rule / this one; us): FP32 137 x 209 x 283 45.0 / 61.9 / 39, 160^3 27.9 /
+// 31.9 / 20, FP64 200^3 69 / 58 / 46.
+// FP64 27-point kernels with 2 rows fit four workgroups a CU: a few more than 1024
+// leave the last ones nearly alone, so the chunk grows until they fit (65 x 129 x
+// 257, apply, 8 planes 23.0, 9 planes 18.3; 160^3 residual 37.6, 10 planes 33).
+static ZCfg default_cfg(int kind, int mode, int dtype, const Box3& ibox)
 {
     ZCfg c;
-    c.ry = (box_nz(ibox) >= 16 || dtype == PM_F32) && zblocks(ibox, 4, 16) >= 768 ? 4
-                                                                                   : (zblocks(ibox, 2, 4) >= 512 ? 2 : 1);
+    const long nz = box_nz(ibox);
+    c.ry = (nz >= 16 || dtype == PM_F32) && zblocks(ibox, 4, 16) >= 768 ? 4 : (zblocks(ibox, 2, 4) >= 512 ? 2 : 1);
+    c.tz = 0;
+    if (kind == 1 && nz > 1) {
+        c.ry = zblocks(ibox, 4, 4) >= 512 ? 4 : (zblocks(ibox, 2, 4) >= 512 ? 2 : 1);
+        c.tz = zblocks(ibox, 4, 8) >= 2048 ? 8 : 4;
+        while (zblocks(ibox, c.ry, c.tz) > 16384 && c.tz < nz) { c.tz *= 2; }
+    } else if (kind % 100 == 27 && dtype == PM_F64 && c.ry == 2) {
+        const int tz = (int)std::min<long>(auto_tz(ibox, 2), nz);
+        const long most = 1024, blocks = zblocks(ibox, 2, tz);
+        if (blocks > most && blocks <= most + most / 4) {
+            c.tz = tz;
+            while (zblocks(ibox, 2, c.tz) > most && c.tz < nz) { c.tz++; }
+        }
+    }
     c.pf = c.ry == 4 || mode >= ZM_RESIDUAL ? 1 : 2;
     c.nt = box_size(ibox) * (long)dtype_size(dtype) >= 32L << 20 ? 1 : 0;
-    c.tz = 0;
     return c;
 }
 
@@ -847,7 +867,7 @@ static ZCfg lookup_cfg(int kind, int mode, int dtype, const Box3& ib)
         auto it = g_tune->find(tune_key(kind, mode, dtype, ib));
         if (it != g_tune->end()) { return it->second; }
     }
-    return default_cfg(mode, dtype, ib);
+    return default_cfg(kind, mode, dtype, ib);
 }
 
 static void store_cfg(const TuneKey& k, const ZCfg& c)
@@ -1200,7 +1220,7 @@ static int autotune_t(const pm_stencil* st, const pm_stencil* st2, int mode, con
     const int nz = (int)box_nz(ib);
     const int tzs[6] = {0, 16, 32, 64, 128, 256};
     float bms = 1e30f;
-    ZCfg bc = default_cfg(mode, dtype_of<T>::value, ib);
+    ZCfg bc = default_cfg(key_kind(st, st2, mode), mode, dtype_of<T>::value, ib);
     for (int ry : kRY)
         for (int pf = 1; pf <= 2; pf++)
             for (int nt = 0; nt <= 1; nt++)
