@@ -107,8 +107,9 @@ static bool covers_periodic(const pm_layout* L)
            L->periodic[2];
 }
 
-// Largest level: the block passes recompute 2.8 times the updates (FP64 tiles
-// leave one workgroup a CU), so they pay while launches and latency dominate.
+// Largest level: on 16 x 8 x 8 tiles the pass down does 3.7 times the updates, the one
+// up 2.4 times (more on thinner tiles), and FP64 tiles leave one workgroup a CU, so
+// they pay while launches and latency dominate.
 // us of one V-cycle solve (10 cycles) with every level of up to 64^3 / 96^3 /
 // 128^3 cells swept this way: FP32 cycles, 32^3 boxes, 128^3 cells: 2660 / 2667
 // / 2413; 64^3 boxes (whose sweeps run the row-register kernels) 1752 / 1773 /

@@ -76,10 +76,11 @@ __global__ __launch_bounds__(256) void k_exchange(LayoutDev L, G3 g, T* data, in
 
 // The same where no ghost layer is wider than a box and a box has fewer than 2^20
 // ghost cells: the 27 neighbouring boxes are looked up once per workgroup and cell
-// positions come from float reciprocals.  Large exchanges are bound by the partial
-// lines of the x and y faces (a 4-cell x face of FP64 moves 32 of each 128-byte
-// line): 540 MB in 173 -> 167 us.  Small ones by the index arithmetic of the general
-// kernel (64-bit divisions a cell): 32^3 boxes, FP32 x 3, 9.4 -> 6.0 us.
+// positions come from float reciprocals.  Large exchanges are bound by the small
+// pieces of the x and y faces (a 4-cell x face of FP64 is 32 bytes of a 128-byte
+// line): 540 MB in 173 -> 167 us, with little more HBM traffic than that (303 MB
+// read, 270 MB written).  Small ones by the index arithmetic of the general kernel
+// (64-bit divisions a cell): 32^3 boxes, FP32 x 3, 9.4 -> 6.0 us.
 template<typename T>
 __global__ __launch_bounds__(256) void k_exchange_nb(LayoutDev L, G3 g, T* data, int ncomp)
 {

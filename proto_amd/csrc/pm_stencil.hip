@@ -613,8 +613,9 @@ __global__ __launch_bounds__(256) void k_zgen(ZArgs<T> a)
 }
 
 // The one-block second stage of k_zgen's reductions (fixed strided split and tree
-// for a count of partials).  As many threads as partials, whole waves, at most 1024:
-// a 256^2 apply + absMax 9.2 -> 7.5 us against always 1024.
+// for a count of partials).  As many threads as partials, whole waves, at most 1024
+// (a 256^2 apply + absMax takes 9.2 us so and with 1024 threads: the launch is what
+// it waits for).
 template<typename T>
 __global__ __launch_bounds__(1024) void k_finish_op(int op, const T* __restrict__ partials, int nb, T* out,
                                                     int combine)
@@ -784,8 +785,8 @@ static long zblocks(const Box3& ibox, int ry, int tz)
 // stage less halo (a run of tz stages tz + 2 planes), short ones reach all 256
 // CUs and end sooner (a plane takes a few hundred ns of load latency and
 // barriers).  16 from about 460^3 cells on, 8 while that leaves four workgroups a
-// CU, else 4; more than 16 only to keep the count
-// of workgroups (and their partials) bounded.
+// CU, else 4; more than 16 only to keep the count of workgroups (and their
+// partials) bounded.
 static int auto_tz(const Box3& ibox, int ry)
 {
     if (zblocks(ibox, ry, 16) >= 6000) {
@@ -801,9 +802,10 @@ static int auto_tz(const Box3& ibox, int ry)
 // ahead where there are few rows to load a plane (not in the residuals, which
 // hold f too).  Non-temporal stores where the result would not stay in cache
 // anyway (200^3 FP64, three arrays in turn: 38.8 -> 21.5 us).  Every configuration
-// was timed over cubes of 48..512 cells and boxes such as 137 x 209 x 283; this
-// rule is within 10 % of the best of nearly all.  Against the fixed shape before
-// it (2 rows in FP64, 4 in FP32, cached stores, 16 planes or more; us):
+// was timed on 27 boxes, cubes of 24..400 cells and thin and ragged ones: the rule's
+// mean is within 4 to 11 % of the best of each operator.  Against the fixed shape
+// before it (2 rows in FP64, 4 in FP32, cached stores, 16 planes or more; us; flat
+// boxes such as 512 x 512 x 16 lose up to 15 % to it when they accumulate):
 //                    64^3          160^3         512^3
 //   7-point FP64     7.1 ->  5.6   14.4 -> 13.5  431 -> 387
 //   27-point FP64   10.0 ->  5.5   20.0 -> 20.2  450 -> 388
